@@ -69,6 +69,19 @@ def test_jaccard_bit_exact(B, n, m, d):
     assert_equal(got, torch.from_numpy(want_c), "jaccard vs C passes")
 
 
+# rows of at most 8 words and m % 4 != 0: the 32 x 512 tile with dword row stores, at the edges of
+# its column groups (64), tile width (512) and rows (32), with and without row popcounts
+@pytest.mark.parametrize("m", [257, 319, 321, 511, 513, 1089])
+@pytest.mark.parametrize("B,n,d", [(1, 1, 1), (2, 33, 166), (1, 64, 256)])
+def test_bool_ragged_rows_bit_exact(B, n, m, d):
+    x1, x2 = rand(B, n, d, seed=7) < 0.4, rand(B, m, d, seed=8) < 0.4
+    x2[:, :3] = False
+    got = capi.bool_pairwise_reduce(x1.to(DEV), x2.to(DEV), capi.BIT_EQ, capi.RED_MEAN)
+    assert_equal(got, torch.from_numpy(P.pw_reduce_bool(x1.numpy(), x2.numpy(), "eq", "mean")), f"eq mean m={m}")
+    assert_equal(capi.jaccard_bool(x1.to(DEV), x2.to(DEV)),
+                 torch.from_numpy(P.jaccard_distances(x1.numpy(), x2.numpy())), f"jaccard m={m}")
+
+
 def test_bool_empty_sizes():
     x1 = torch.zeros((0, 16), dtype=torch.bool, device=DEV)
     x2 = torch.zeros((5, 16), dtype=torch.bool, device=DEV)

@@ -256,7 +256,12 @@ __device__ __forceinline__ uint32_t popacc(uint32_t acc, uint4 a, uint4 b) {
 // CV uint4 (4 words) per row and LDS chunk.  128 x 128 (TX = 16) for general rows; 32 x 512
 // (TX = 64) for rows of at most 8 words, where the output write is the whole cost and 2 KB
 // contiguous per row and tile keep the DRAM pages open longer than 512 B.
-template <int OP, int EPI, int TX, int CV>
+// RAGGED (TX = 64, rows of m % 4 != 0 floats or an unaligned output, which no 16-byte store
+// fits): thread tx owns columns tx + 64 j instead, so each dword store instruction of a wave
+// covers 256 contiguous bytes of one row; in the aligned column order its lanes would be 16
+// bytes apart and every line written in four passes (hamming 2000 x 30011 x 166: 300 -> 84 us
+// a call).
+template <int OP, int EPI, int TX, int CV, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
     const uint32_t *__restrict__ A, const uint32_t *__restrict__ Bw,
     const int32_t *__restrict__ popA, const int32_t *__restrict__ popB, int64_t n, int64_t m,
@@ -266,6 +271,8 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
     __shared__ uint4 As[RT][CV + 1];
     __shared__ uint4 Bs[CT][CV + 1];
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
+    // tile column of the thread's j-th output
+    auto tile_col = [tx](int j) { return RAGGED ? tx + TX * j : (j >> 2) * (4 * TX) + 4 * tx + (j & 3); };
     const int64_t b = blockIdx.z;
     const int64_t row0 = (int64_t)blockIdx.y * RT, col0 = (int64_t)blockIdx.x * CT;
     const uint32_t *Ab = A + b * n * W;
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i) a[i] = As[ty + TY * i][c];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bv[j] = Bs[(j >> 2) * (4 * TX) + 4 * tx + (j & 3)][c];
+            for (int j = 0; j < 8; ++j) bv[j] = Bs[tile_col(j)][c];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -316,6 +323,17 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
         uint32_t pa = 0;
         if constexpr (kPops) pa = (uint32_t)popA[b * n + row];
         const float df = (float)d;
+        if constexpr (RAGGED) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int64_t col = col0 + tile_col(j);
+                uint32_t pb = 0;
+                if constexpr (kPops) pb = col < m ? (uint32_t)popB[b * m + col] : 0u;
+                const float v = finish<OP, EPI>(acc[i][j], pa, pb, (uint32_t)d, inv_d, df, inv_df);
+                if (col < m) orow[col] = v;
+            }
+            continue;
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int64_t col = col0 + 4 * TX * h + 4 * tx;
@@ -348,7 +366,11 @@ int launch_reduce(const uint32_t *a, const uint32_t *b, const int32_t *pa, const
     const LaunchEvents ev = launch_events("bool_reduce_kernel");
     if (W <= 8 && m > 256 && cdiv(n, 32) <= kMaxGridYZ) {
         dim3 grid((unsigned)cdiv(m, 512), (unsigned)cdiv(n, 32), (unsigned)batch);
-        hipExtLaunchKernelGGL((bool_reduce_kernel<OP, EPI, 64, 2>), grid, dim3(kThreads), 0, s, ev.start, ev.stop, 0, a, b,
+        if (!vec_store)
+            hipExtLaunchKernelGGL((bool_reduce_kernel<OP, EPI, 64, 2, true>), grid, dim3(kThreads), 0, s, ev.start,
+                                  ev.stop, 0, a, b, pa, pb, n, m, W, d, inv_d, inv_df, out, vec_store);
+        else
+            hipExtLaunchKernelGGL((bool_reduce_kernel<OP, EPI, 64, 2>), grid, dim3(kThreads), 0, s, ev.start, ev.stop, 0, a, b,
                            pa, pb, n, m, W, d, inv_d, inv_df, out, vec_store);
     } else {
         dim3 grid((unsigned)cdiv(m, kTile), (unsigned)cdiv(n, kTile), (unsigned)batch);
