@@ -196,6 +196,27 @@ def _sign_counts(a, b):
     return np.nan_to_num(np.sign(diff), nan=0.0).sum(axis=1)
 
 
+# splits of one 32-pair stage (few output rows against many), their count capped, a last split of
+# one pair, and grids whose splits are more stages long
+@pytest.mark.parametrize("p", [1.0, 1.5, 3.0])
+@pytest.mark.parametrize("B,n,m,d", [(1, 3, 33, 9), (1, 64, 1569, 16), (2, 129, 2081, 65), (1, 40, 4100, 128),
+                                     (3, 1000, 65, 70)])
+def test_lp_backward_short_splits(p, B, n, m, d):
+    from tests import _gradbound as GB
+
+    x1, x2, g = randn(B, n, d, seed=31), randn(B, m, d, seed=32), randn(B, n, m, seed=33)
+    dist = capi.lp_distances(x1.to(DEV), x2.to(DEV), p)
+    got = capi.lp_distances_backward2(g.to(DEV), x1.to(DEV), x2.to(DEV), dist, p)
+    diff = x1.double()[:, :, None, :] - x2.double()[:, None, :, :]
+    dd = diff.abs().pow(p).sum(-1).pow(1.0 / p)
+    terms = diff.sign() * diff.abs().pow(p - 1.0) * (g.double() / dd.pow(p - 1.0))[..., None]
+    # a term: the weight (p = 1.5, 3: the distance's error times p - 1, a divide), the hardware
+    # log2 / exp2 of a fractional power, two products
+    c_t = {1.0: 1.0, 1.5: 24.0, 3.0: 12.0}[p]
+    GB.check(got[0].cpu(), terms.sum(2), GB.sum_bound(terms, 2, c_t), f"grad_x1 p={p}")
+    GB.check(got[1].cpu(), -terms.sum(1), GB.sum_bound(terms, 1, c_t), f"grad_x2 p={p}")
+
+
 @pytest.mark.parametrize("entry", ["single", "both"])
 def test_lp_backward_p1_sign_exact(entry):
     """p = 1 with grad = 1: every gradient is an integer count, exact in fp32, so the

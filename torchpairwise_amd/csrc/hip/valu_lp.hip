@@ -986,7 +986,15 @@ __global__ void sum_splits_kernel(const float *__restrict__ part, int64_t splits
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= len) return;
     float s = part[t];
-    for (int64_t q = 1; q < splits; ++q) s += part[q * len + t];
+    int64_t q = 1;
+    for (; q + 8 <= splits; q += 8) {  // eight loads in flight, added in split order
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = part[(q + e) * len + t];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += v[e];
+    }
+    for (; q < splits; ++q) s += part[q * len + t];
     out[t] = s;
 }
 
@@ -1141,18 +1149,23 @@ int device_cus() {
 
 // Number of j splits for `slots` resident blocks: the (row block, feature block, batch)
 // grid alone fills base blocks; splitting j multiplies that, and a whole number of
-// resident rounds avoids a partly filled last round.  More slots never give fewer splits,
-// so the workspace is sized with the largest slot count.
+// resident rounds avoids a partly filled last round.  A split is a whole number of kBJ-pair
+// stages, down to one: a block of few stages costs about 5 us a stage while its SIMDs hold one
+// wave each, so a small problem is as long as its longest split, and the partials of `slots`
+// blocks (32 or 64 KB each) take a few us to add (manhattan forward and backward 3001 x 1999 x
+// 100: 368 -> 200 us against splits of at least 512 pairs; 3176 x 3178 x 10: 328 -> 120).  More slots never give fewer splits, so the
+// workspace is sized with the largest slot count.
+constexpr int64_t kMaxSplits = 64;
 int64_t lp_backward_splits(int64_t slots, int64_t batch, int64_t n, int64_t m, int64_t d, int64_t fw) {
     const int64_t base = cdiv(n, kBRows) * cdiv(d, fw) * batch;
-    if (base == 0) return 1;  // no output rows (empty n, d or batch): nothing to split
+    if (base == 0 || m == 0) return 1;  // nothing to split
     int64_t splits = base >= slots ? 1 : slots / base;
-    const int64_t max_by_m = cdiv(m, 512);
-    if (splits > max_by_m) splits = max_by_m;
-    if (splits > 16) splits = 16;
+    if (splits > kMaxSplits) splits = kMaxSplits;
+    if (splits * batch > kMaxGridYZ) splits = kMaxGridYZ / batch;
     if (splits < 1) splits = 1;
-    while (splits > 1 && splits * batch > kMaxGridYZ) --splits;
-    return splits;
+    // whole stages per split, then only as many splits as hold pairs
+    const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
+    return cdiv(m, jps);
 }
 int64_t max_slots() { return (int64_t)device_cus() * kMaxBlocksPerCU; }
 
