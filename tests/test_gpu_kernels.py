@@ -170,6 +170,20 @@ def test_lp_forward(p, B, n, m, d):
     assert_close(got, want, rtol=1e-5, atol=1e-6 * float(want.abs().max()), what=f"lp p={p}")
 
 
+# 64 x 64 tiles (grids of fewer 128 x 128 tiles than 7/4 of the CUs) against 128 x 128 tiles (the
+# same rows inside a batch of 460): each output's sum runs in the same order, so the bits agree.
+# Edges of both tiles, full and ragged rows (m % 4), whole and ragged feature chunks (d % 4, d % 32).
+@pytest.mark.parametrize("n,m,d", [(64, 64, 32), (65, 63, 37), (1, 129, 3), (128, 66, 33), (31, 60, 100)])
+@pytest.mark.parametrize("p", [0.0, 1.0, 1.5, 2.0, 3.0, 4.5, float("inf")])
+def test_lp_forward_tile_sizes_agree(p, n, m, d):
+    x1, x2 = randn(460, n, d, seed=41).to(DEV), randn(460, m, d, seed=42).to(DEV)
+    for fn in (lambda a, b: capi.lp_distances(a, b, p), lambda a, b: capi.lp_distances_bf16(a, b, p),
+               lambda a, b: capi.family_forward(capi.FAM_PPMINKOWSKI, a, b, p=p)):
+        whole = fn(x1, x2)
+        for b in (0, 459):
+            assert_equal(fn(x1[b:b + 1], x2[b:b + 1])[0], whole[b], f"p={p} batch {b}")
+
+
 @pytest.mark.parametrize("p", [1.0, 1.5, 2.0, 3.0, 4.5, float("inf")])
 @pytest.mark.parametrize("B,n,m,d", [(1, 130, 200, 64), (2, 40, 33, 5), (1, 700, 1100, 70), (1, 7, 9, 5),
                                      (1, 300, 257, 128), (2, 65, 130, 200)])

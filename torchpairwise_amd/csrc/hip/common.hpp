@@ -34,6 +34,7 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 constexpr int64_t kMaxGridYZ = 65535;
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // at a dword-aligned address
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -114,8 +115,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_over(const float *base,
 __device__ __forceinline__ float buffer_load(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset) {
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)byte_offset, 0, 0));
 }
-// Four floats at a 16-byte aligned byte offset (whole in range or whole out: the caller keeps
-// array lengths and offsets multiples of 4 floats).
+// Four floats at a dword-aligned byte offset, all of them in range.
 typedef unsigned int tpw_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ floatx4 buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset) {
     return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte_offset, 0, 0));

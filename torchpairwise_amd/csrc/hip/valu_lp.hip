@@ -183,53 +183,70 @@ __device__ __forceinline__ float fam_finish(float acc, float inv_p, float prev) 
 template <int PK>
 constexpr int kFwdBlocks = (PK == kPInf || PK == kPNInf) ? 3 : 2;
 
-template <int MODE, int PK, bool VEC, int OM = 0>
+// TT: rows and columns of the output tile, 128 (8 x 8 outputs a thread) or, where those tiles
+// would not fill the GPU, 64 (4 x 4 outputs): four times the blocks, each a quarter as long, for
+// twice the LDS reads per pair-feature.  An output's sum runs over k in the same order in both.
+template <int MODE, int PK, bool VEC, int OM = 0, int TT = kTile>
 __global__ __launch_bounds__(kThreads, kFwdBlocks<PK>) void lp_forward_kernel(
     const float *__restrict__ x1, const float *__restrict__ x2, const float *__restrict__ w,
     int64_t n, int64_t m, int64_t d, float p, float inv_p, float *__restrict__ out, float post,
     const float *__restrict__ rownum, uint16_t *__restrict__ out16) {
-    __shared__ float As[kBK][kTile + kPad];
-    __shared__ float Bs[kBK][kTile + kPad];
+    static_assert(TT == 128 || TT == 64, "tile size");
+    constexpr int R = TT / 16;  // rows and columns per thread
+    __shared__ float panels[2][kBK][TT + kPad];
+    auto &As = panels[0];
+    auto &Bs = panels[1];
     __shared__ float Wk[MODE == kWeighted ? kBK : 1];
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     const int64_t b = blockIdx.z;
-    const int64_t row0 = (int64_t)blockIdx.y * kTile, col0 = (int64_t)blockIdx.x * kTile;
+    const int64_t row0 = (int64_t)blockIdx.y * TT, col0 = (int64_t)blockIdx.x * TT;
     const float *A = x1 + b * n * d;
     const float *B = x2 + b * m * d;
 
-    float acc[8][8];
+    float acc[R][R];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = fam_init<MODE, PK>();
+        for (int j = 0; j < R; ++j) acc[i][j] = fam_init<MODE, PK>();
 
-    // staging: 128 rows x 32 features per operand = 1024 float4, 4 per thread
-    auto load = [&](const float *X, int64_t rows, int64_t r0, int64_t k0, floatx4 (&v)[4]) {
+    // staging: TT rows x 32 features per operand, R / 2 float4 per thread
+    auto load = [&](const float *X, int64_t rows, int64_t r0, int64_t k0, floatx4 (&v)[R / 2]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < R / 2; ++q) {
             const int idx = tid + kThreads * q;
             const int r = idx >> 3, c4 = idx & 7;
             const int64_t gr = r0 + r, gk = k0 + 4 * c4;
             floatx4 t = {0.0f, 0.0f, 0.0f, 0.0f};
             if (gr < rows) {
                 const float *src = X + gr * d + gk;
-                if constexpr (VEC) {
-                    if (gk < d) t = *reinterpret_cast<const floatx4 *>(src);
-                } else {
+                if (VEC ? gk < d : gk + 3 < d) {
+                    // !VEC: a 16-byte load at a dword-aligned address, which global memory allows
+                    t = VEC ? *reinterpret_cast<const floatx4 *>(src) : *reinterpret_cast<const floatx4u *>(src);
+                } else if constexpr (!VEC) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
+                    for (int e = 0; e < 3; ++e)
                         if (gk + e < d) t[e] = src[e];
                 }
             }
             v[q] = t;
         }
     };
-    floatx4 pa[4], pb[4];
+    floatx4 pa[R / 2], pb[R / 2];
+    // the thread's R row and R column values of step k
+    auto read_step = [&](float (&av)[R], float (&bv)[R], int k) {
+#pragma unroll
+        for (int h = 0; h < R / 4; ++h) {
+            const floatx4 a = *reinterpret_cast<const floatx4 *>(&As[k][R * ty + 4 * h]);
+            const floatx4 c = *reinterpret_cast<const floatx4 *>(&Bs[k][64 * h + 4 * tx]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) av[4 * h + e] = a[e], bv[4 * h + e] = c[e];
+        }
+    };
     load(A, n, row0, 0, pa);
     load(B, m, col0, 0, pb);
     for (int64_t k0 = 0; k0 < d; k0 += kBK) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < R / 2; ++q) {
             const int idx = tid + kThreads * q;
             const int r = idx >> 3, c4 = idx & 7;
 #pragma unroll
@@ -250,48 +267,34 @@ __global__ __launch_bounds__(kThreads, kFwdBlocks<PK>) void lp_forward_kernel(
         int kbeg = 0;
         if constexpr ((PK == kPInf || PK == kPNInf) && (MODE == kRoot || MODE == kSum)) {
             for (; kbeg + 1 < kmax; kbeg += 2) {
-                float av[2][8], bv[2][8];
+                float av[2][R], bv[2][R];
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const floatx4 a0 = *reinterpret_cast<const floatx4 *>(&As[kbeg + h][8 * ty]);
-                    const floatx4 a1 = *reinterpret_cast<const floatx4 *>(&As[kbeg + h][8 * ty + 4]);
-                    const floatx4 b0 = *reinterpret_cast<const floatx4 *>(&Bs[kbeg + h][4 * tx]);
-                    const floatx4 b1 = *reinterpret_cast<const floatx4 *>(&Bs[kbeg + h][64 + 4 * tx]);
+                for (int h = 0; h < 2; ++h) read_step(av[h], bv[h], kbeg + h);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        av[h][e] = a0[e], av[h][4 + e] = a1[e];
-                        bv[h][e] = b0[e], bv[h][4 + e] = b1[e];
-                    }
-                }
+                for (int i = 0; i < R; ++i)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
+                    for (int j = 0; j < R; ++j) {
                         const float d0 = av[0][i] - bv[0][j], d1 = av[1][i] - bv[1][j];
                         acc[i][j] = PK == kPInf ? max3_abs(acc[i][j], d0, d1) : min3_abs(acc[i][j], d0, d1);
                     }
             }
         }
         for (int k = kbeg; k < kmax; ++k) {
-            const floatx4 a0 = *reinterpret_cast<const floatx4 *>(&As[k][8 * ty]);
-            const floatx4 a1 = *reinterpret_cast<const floatx4 *>(&As[k][8 * ty + 4]);
-            const floatx4 b0 = *reinterpret_cast<const floatx4 *>(&Bs[k][4 * tx]);
-            const floatx4 b1 = *reinterpret_cast<const floatx4 *>(&Bs[k][64 + 4 * tx]);
+            float av[R], bv[R];
+            read_step(av, bv, k);
             const float wk = MODE == kWeighted ? Wk[MODE == kWeighted ? k : 0] : 0.0f;
-            const float av[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-            const float bv[8] = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
             if constexpr ((MODE == kRoot || MODE == kSum) && (PK == kP1 || PK == kP2)) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < R; ++i)
 #pragma unroll
-                    for (int j = 0; j < 8; j += 4)
+                    for (int j = 0; j < R; j += 4)
                         lp_step4<PK>(acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3], av[i], bv[j], bv[j + 1],
                                      bv[j + 2], bv[j + 3]);
             } else {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < R; ++i)
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) acc[i][j] = fam_step<MODE, PK>(acc[i][j], av[i], bv[j], wk, p);
+                    for (int j = 0; j < R; ++j) acc[i][j] = fam_step<MODE, PK>(acc[i][j], av[i], bv[j], wk, p);
             }
         }
         __syncthreads();
@@ -300,19 +303,19 @@ __global__ __launch_bounds__(kThreads, kFwdBlocks<PK>) void lp_forward_kernel(
     const bool vec_store = VEC && (m % 4 == 0);
     if (!vec_store) {
         // rows of m % 4 != 0 floats (or unaligned outputs): the tile goes through the operand
-        // LDS (free after the K loop's last barrier) in four 64 x 64 quarters, and each wave
+        // LDS (free after the K loop's last barrier) in 64 x 64 pieces, and each wave
         // writes whole 64-value row pieces, a dword per lane: 256 contiguous bytes per store
         // instead of 4-byte stores 16 bytes apart
         constexpr int kSt = 66;
-        static_assert(64 * kSt <= kBK * (kTile + kPad), "the stage fits in As");
-        float *st = &As[0][0];
+        static_assert(64 * kSt <= 2 * kBK * (TT + kPad), "the stage fits in the panels");
+        float *st = &panels[0][0][0];
         const int wave = tid >> 6, lane = tid & 63;
-        for (int rh = 0; rh < 2; ++rh)
-            for (int h = 0; h < 2; ++h) {
-                if ((ty >> 3) == rh) {
+        for (int rh = 0; rh < R / 4; ++rh)
+            for (int h = 0; h < R / 4; ++h) {
+                if (R * ty / 64 == rh) {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const int64_t row = row0 + 8 * ty + i;
+                    for (int i = 0; i < R; ++i) {
+                        const int64_t row = row0 + R * ty + i;
                         const int64_t col = col0 + 64 * h + 4 * tx;
                         floatx4 prev = {0.0f, 0.0f, 0.0f, 0.0f};
                         if constexpr (MODE == kBrayDen) {
@@ -334,7 +337,7 @@ __global__ __launch_bounds__(kThreads, kFwdBlocks<PK>) void lp_forward_kernel(
                             for (int c = 0; c < 4; ++c) v[c] = __fdiv_rn(num, v[c]);
                         }
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) st[(8 * ty + i - 64 * rh) * kSt + 4 * tx + c] = v[c];
+                        for (int c = 0; c < 4; ++c) st[(R * ty + i - 64 * rh) * kSt + 4 * tx + c] = v[c];
                     }
                 }
                 __syncthreads();
@@ -352,12 +355,12 @@ __global__ __launch_bounds__(kThreads, kFwdBlocks<PK>) void lp_forward_kernel(
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int64_t row = row0 + 8 * ty + i;
+    for (int i = 0; i < R; ++i) {
+        const int64_t row = row0 + R * ty + i;
         if (row >= n) continue;
         float *orow = out + (b * n + row) * m;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < R / 4; ++h) {
             const int64_t col = col0 + 64 * h + 4 * tx;
             floatx4 prev = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (MODE == kBrayDen) {
@@ -631,7 +634,9 @@ __global__ void pair_weight_kernel(const float *__restrict__ g, const float *__r
 // backward, so no N x M pass forms that gradient first.  gate: when not null, the block runs
 // only if *gate == gate_run (two instances of one backward launched together, a flag set by an
 // earlier launch choosing which one computes).
-template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW = kBFeat, bool EXPG = false>
+// WHOLE: n, m and d are multiples of 4 (and the staging offsets 32-bit), so each 16-byte staging
+// load lies whole in its array or whole past its end, where it reads 0, and needs no test.
+template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW = kBFeat, bool EXPG = false, bool WHOLE = false>
 __global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
     const float *__restrict__ g, const float *__restrict__ aux0, const float *__restrict__ aux1,
     const float *__restrict__ x1, const float *__restrict__ x2, const float *__restrict__ w,
@@ -641,7 +646,6 @@ __global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
     if (gate != nullptr && __builtin_amdgcn_readfirstlane(*gate) != gate_run) return;
     constexpr bool kTwo = (MODE == kRoot && PK == kPInf) || MODE == kBrayDen;
     constexpr int kCW = FW / 16;                // features per thread
-    constexpr int kWavesPerRow = FW / 64;       // waves staging one x2 panel row
     constexpr int kPanelQ = kBJ * FW / kThreads;  // x2 panel values per thread and stage
     static_assert(FW == 64 || FW == 128, "feature width");
     __shared__ float Ws[kBJ][kBRows + kPad];
@@ -680,15 +684,17 @@ __global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
 
     // Staging is software-pipelined: the per-pair values and the x2 panel of stage j0 + kBJ
     // are loaded into registers while stage j0 is computed from LDS, and go to LDS after
-    // the stage's closing barrier.  Lane (tid) loads weight q of a stage at
-    //   direct:     row ii = (tid >> 5) + 8 q, column jj = tid & 31   (coalesced along j)
-    //   transposed: row ii = tid & 127,        column jj = (tid >> 7) + 2 q  (along i)
-    // and panel value q at row jj = wave / kWavesPerRow + (4 / kWavesPerRow) q, feature
-    // kk = 64 (wave % kWavesPerRow) + lane.  The loads are
-    // raw buffer loads from wave-uniform bases: a lane past the end of an array reads 0, and
-    // lanes past a row's end (j >= m, k >= d) or past jend read values that only reach
-    // accumulators of rows, features or stage steps that are never stored or run, so no
-    // load needs a bounds branch.
+    // the stage's closing barrier.  Lane (tid) loads four neighbouring values q of a stage at
+    //   direct:     row ii = (tid >> 3) + 32 q, columns jj = 4 (tid & 7) + 0..3
+    //   transposed: column jj = (tid >> 5) + 8 q, rows ii = 4 (tid & 31) + 0..3
+    //   panel:      row jj = tid / (FW / 4) + (1024 / FW) q, features kk = 4 (tid % (FW / 4)) + 0..3
+    // one 16-byte load each
+    // (any dword-aligned address) where the whole stage lies inside the array, else four dword
+    // loads that stop at the array's end.  Values past a row's end (j >= m, k >= d)
+    // or past jend only reach accumulators of rows, features or stage steps that are never stored
+    // or run.  Dword loads throughout cost the narrow
+    // kernel 12 more load instructions per stage, and held the wide one to n, m and d that are
+    // multiples of 4 (rbf 4096 x 4000 x 90, the narrow kernel before: backward 409 -> 230 us).
     constexpr bool kReadG = !PRE;                               // upstream grad
     constexpr bool kReadA0 = PRE || (MODE == kRoot && PK != kP1);  // weights, or the distance
     constexpr bool kReadA1 = PRE && kTwo;
@@ -698,142 +704,101 @@ __global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
         if constexpr (EXPG) return __fmul_rn(__fmul_rn(gv, ev), es);
         else return gv;
     };
-    // The wide kernel (V4) stages with 16-byte loads instead (its launch requires 16-byte
-    // aligned arrays and n, m, d multiples of 4): lane (tid) loads float4 q of a stage at
-    //   direct:     row ii = (tid >> 3) + 32 q, columns jj = 4 (tid & 7) + 0..3
-    //   transposed: column jj = (tid >> 5) + 8 q, rows ii = 4 (tid & 31) + 0..3
-    //   panel:      row jj = (tid >> 5) + 8 q, features kk = 4 (tid & 31) + 0..3
-    // from one descriptor per array and stage with loop-invariant lane offsets.
-    constexpr bool V4 = FW == kBFeatWide;
-    static_assert(!V4 || !kTwo, "the wide kernel stages one per-pair array");
+    constexpr bool kWideFW = FW == kBFeatWide;
+    static_assert(!kWideFW || !kTwo, "the wide kernel stages one per-pair array");
     // The p = 2 power sum on the wide kernel: its terms 2 d g accumulate as d g (the p = 2
     // step of the cdist backward, one fma each) and the sum is doubled once at the end.
     // Doubling is exact, so this differs from summing 2 d g only where a partial sum is
     // subnormal or overflows.
-    constexpr bool kHalfSum = V4 && MODE == kSum && PK == kP2;
+    constexpr bool kHalfSum = kWideFW && MODE == kSum && PK == kP2;
     // p = 1 on the wide kernel: only the pre-scaled sign path (sign_scaled), launched where every
     // value of x1 and x2 lies in the scalable range (sign_range_kernel); x1 is scaled once, the
     // x2 panel as it is staged.  The narrow kernel's per-tile test and its signf path would not
     // fit the wide kernel's registers.
-    constexpr bool kSignOnly = V4 && PK == kP1 && (MODE == kRoot || MODE == kSum) && !WGRAD;
+    constexpr bool kSignOnly = kWideFW && PK == kP1 && (MODE == kRoot || MODE == kSum) && !WGRAD;
     float rg[kReadG ? 16 : 1], ra0[kReadA0 ? 16 : 1], ra1[kReadA1 ? 16 : 1], re[EXPG ? 16 : 1], rx[kPanelQ];
     const int lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lw_i = TR ? (tid & 127) : (tid >> 5), lw_j = TR ? (tid >> 7) : (tid & 31);
-    const int lx_j = (tid >> 6) / kWavesPerRow, lx_k = 64 * ((tid >> 6) % kWavesPerRow) + lane;
-    // byte offsets within a wave's rows (the launch keeps them below 2^32)
-    const uint32_t lw_voff = TR ? (uint32_t)lane * 4u : (uint32_t)(((lane >> 5) * m + (lane & 31)) * 4);
-    const uint32_t lx_voff = (uint32_t)lane * 4u;
+    constexpr int kPanelRow4 = FW / 4;  // lanes per panel row
     const int64_t nm = n * m, md = m * d;
-
-    uint32_t v4_pair_off[V4 ? 4 : 1], v4_panel_off[V4 ? 4 : 1];
-    if constexpr (V4) {
+    const int pair_row = TR ? tid >> 5 : tid >> 3, pair_col = TR ? 4 * (tid & 31) : 4 * (tid & 7);
+    constexpr int kPairStep = TR ? 8 : 32, kPanelStep = kThreads / kPanelRow4;
+    const int panel_row = tid / kPanelRow4, panel_col = 4 * (tid % kPanelRow4);
+    // Q x 4 values: rows row + step q of a stage's array at arr (row stride ld), columns
+    // col .. col + 3; `len` values lie from arr to the array's end, and the stage reaches `span`
+    auto load4 = [&](const float *arr, int64_t len, int64_t span, int64_t ld, int row, int step, int col, auto &r) {
+        constexpr int Q = sizeof(r) / sizeof(floatx4);
+        if (WHOLE || (span <= len && span < ((int64_t)1 << 30))) {  // 32-bit byte offsets
+            const auto rs = buffer_over(arr, len);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v4_pair_off[q] = TR ? (uint32_t)((((tid >> 5) + 8 * q) * n + 4 * (tid & 31)) * 4)
-                                : (uint32_t)((((tid >> 3) + 32 * q) * m + 4 * (tid & 7)) * 4);
-            v4_panel_off[q] = (uint32_t)((((tid >> 5) + 8 * q) * d + 4 * (tid & 31)) * 4);
-        }
-    }
-    // V4: the 16 per-pair values of one array for stage j0, as four float4
-    auto load_pairs4 = [&](const float *arr, auto &r, int64_t j0) {
-        const int64_t off = TR ? j0 * n + i0 : i0 * m + j0;
-        const auto rs = buffer_over(arr + off, nm - off);
+            for (int q = 0; q < Q; ++q) {
+                const floatx4 v = buffer_load4(rs, (uint32_t)((row + step * q) * ld + col) * 4u);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const floatx4 v = buffer_load4(rs, v4_pair_off[q]);
+                for (int e = 0; e < 4; ++e) r[4 * q + e] = v[e];
+            }
+        } else {
+            // opaque to the compiler: the element addresses, invariant over the stages, would
+            // otherwise be formed before the stage loop and spill
+            asm volatile("" : "+v"(row));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[4 * q + e] = v[e];
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int64_t at = (row + step * q) * ld + col + e;
+                    r[4 * q + e] = at < len ? arr[at] : 0.0f;
+                }
         }
     };
     // the 16 per-pair values of one array for stage j0
     auto load_pairs = [&](const float *arr, auto &r, int64_t j0) {
-        // one descriptor per step keeps the lane offset a single register (per-step lane
-        // offsets would be loop-invariant and stay live across the stage loop)
-        if constexpr (TR) {  // 64 rows of one column per wave and step
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int64_t off = (j0 + (wv >> 1) + 2 * q) * n + i0 + (wv & 1) * 64;
-                r[q] = buffer_load(buffer_over(arr + off, nm - off), lw_voff);
-            }
-        } else {  // 32 columns of two rows per wave and step
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int64_t off = (i0 + 2 * wv + 8 * q) * m + j0;
-                r[q] = buffer_load(buffer_over(arr + off, nm - off), lw_voff);
-            }
-        }
+        const int64_t off = TR ? j0 * n + i0 : i0 * m + j0;
+        load4(arr + off, nm - off, TR ? (kBJ - 1) * n + kBRows : (kBRows - 1) * m + kBJ, TR ? n : m, pair_row,
+              kPairStep, pair_col, r);
     };
     auto load = [&](int64_t j0) {
-        if constexpr (V4) {
-            if constexpr (kReadG) load_pairs4(G, rg, j0);
-            if constexpr (kReadA0) load_pairs4(A0, ra0, j0);
-            if constexpr (EXPG) load_pairs4(E, re, j0);
-            const int64_t off = j0 * d + k0;
-            const auto rs = buffer_over(X2 + off, md - off);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const floatx4 v = buffer_load4(rs, v4_panel_off[q]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) rx[4 * q + e] = v[e];
-            }
-            return;
-        }
         if constexpr (kReadG) load_pairs(G, rg, j0);
         if constexpr (kReadA0) load_pairs(A0, ra0, j0);
         if constexpr (kReadA1) load_pairs(A1, ra1, j0);
         if constexpr (EXPG) load_pairs(E, re, j0);
-#pragma unroll
-        for (int q = 0; q < kPanelQ; ++q) {
-            const int64_t off = (j0 + wv / kWavesPerRow + (4 / kWavesPerRow) * q) * d + k0 + 64 * (wv % kWavesPerRow);
-            rx[q] = buffer_load(buffer_over(X2 + off, md - off), lx_voff);
-        }
+        const int64_t off = j0 * d + k0;
+        load4(X2 + off, md - off, (kBJ - 1) * d + FW, d, panel_row, kPanelStep, panel_col, rx);
     };
     auto store = [&](int64_t j0) {
-        if constexpr (V4) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float wq[4];
+        for (int q = 0; q < 4; ++q) {
+            float wq[4], dq[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int ii = TR ? 4 * (tid & 31) + e : (tid >> 3) + 32 * q;
+                const int jj = TR ? (tid >> 5) + 8 * q : 4 * (tid & 7) + e;
+                float w1, w2;
+                if constexpr (PRE) {
+                    w1 = ra0[4 * q + e];
+                    w2 = kTwo ? ra1[kTwo ? 4 * q + e : 0] : 0.0f;
+                } else {
+                    pair_weights<MODE, PK>(gval(rg[4 * q + e], re[EXPG ? 4 * q + e : 0]),
+                                           kReadA0 ? ra0[kReadA0 ? 4 * q + e : 0] : 0.0f, 0.0f, p, w1, w2);
+                }
+                const bool in = i0 + ii < n && j0 + jj < jend;
+                wq[e] = in ? w1 : 0.0f;
+                dq[e] = in ? w2 : 0.0f;
+            }
+            if constexpr (TR) {
+                const int jj = (tid >> 5) + 8 * q, ii = 4 * (tid & 31);
+                *reinterpret_cast<floatx4 *>(&Ws[jj][ii]) = floatx4{wq[0], wq[1], wq[2], wq[3]};
+                if constexpr (kTwo) *reinterpret_cast<floatx4 *>(&Ds[jj][ii]) = floatx4{dq[0], dq[1], dq[2], dq[3]};
+            } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int ii = TR ? 4 * (tid & 31) + e : (tid >> 3) + 32 * q;
-                    const int jj = TR ? (tid >> 5) + 8 * q : 4 * (tid & 7) + e;
-                    float w1, w2;
-                    pair_weights<MODE, PK>(kReadG ? gval(rg[4 * q + e], re[EXPG ? 4 * q + e : 0]) : 0.0f,
-                                           kReadA0 ? ra0[4 * q + e] : 0.0f, 0.0f, p, w1, w2);
-                    if constexpr (PRE) w1 = ra0[4 * q + e];
-                    wq[e] = (i0 + ii < n && j0 + jj < jend) ? w1 : 0.0f;
-                }
-                if constexpr (TR) {
-                    *reinterpret_cast<floatx4 *>(&Ws[(tid >> 5) + 8 * q][4 * (tid & 31)]) =
-                        floatx4{wq[0], wq[1], wq[2], wq[3]};
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) Ws[4 * (tid & 7) + e][(tid >> 3) + 32 * q] = wq[e];
-                }
-                const float sc = kSignOnly ? kSignScale : 1.0f;  // exact in the scalable range
-                *reinterpret_cast<floatx4 *>(&Xs[(tid >> 5) + 8 * q][4 * (tid & 31)]) =
-                    floatx4{rx[4 * q] * sc, rx[4 * q + 1] * sc, rx[4 * q + 2] * sc, rx[4 * q + 3] * sc};
-            }
-            return;
-        }
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int ii = lw_i + (TR ? 0 : 8 * q), jj = lw_j + (TR ? 2 * q : 0);
-            float w1 = 0.0f, w2 = 0.0f;
-            if (i0 + ii < n && j0 + jj < jend) {
-                if constexpr (PRE) {
-                    w1 = ra0[q];
-                    if constexpr (kTwo) w2 = ra1[q];
-                } else {
-                    pair_weights<MODE, PK>(gval(rg[q], re[EXPG ? q : 0]), kReadA0 ? ra0[q] : 0.0f, 0.0f, p, w1, w2);
+                    Ws[4 * (tid & 7) + e][(tid >> 3) + 32 * q] = wq[e];
+                    if constexpr (kTwo) Ds[4 * (tid & 7) + e][(tid >> 3) + 32 * q] = dq[e];
                 }
             }
-            Ws[jj][ii] = w1;
-            if constexpr (kTwo) Ds[jj][ii] = w2;
         }
+        const float sc = kSignOnly ? kSignScale : 1.0f;  // exact in the scalable range
 #pragma unroll
-        for (int q = 0; q < kPanelQ; ++q) Xs[lx_j + (4 / kWavesPerRow) * q][lx_k] = rx[q];
+        for (int q = 0; q < kPanelQ / 4; ++q)
+            *reinterpret_cast<floatx4 *>(&Xs[(tid / kPanelRow4) + (kThreads / kPanelRow4) * q][4 * (tid % kPanelRow4)]) =
+                floatx4{rx[4 * q] * sc, rx[4 * q + 1] * sc, rx[4 * q + 2] * sc, rx[4 * q + 3] * sc};
     };
 
     // x2 values of panel row jj at the thread's features feat_of(tcol, c) (one or two 16-byte
@@ -1065,6 +1030,14 @@ __global__ void fill_kernel(float *__restrict__ p, int64_t len, float v) {
     if (t < len) p[t] = v;
 }
 
+int device_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return 256;
+    return cus;
+}
+
 int pkind_of(double p) {
     if (p == 0.0) return kP0;
     if (p == 1.0) return kP1;
@@ -1079,18 +1052,31 @@ template <int MODE, int PK>
 int launch_forward(const float *x1, const float *x2, const float *w, int64_t batch, int64_t n,
                    int64_t m, int64_t d, double p, float *out, hipStream_t s, bool exp_post = false,
                    float post = 0.0f, const float *rownum = nullptr, uint16_t *out16 = nullptr) {
-    dim3 grid((unsigned)cdiv(m, kTile), (unsigned)cdiv(n, kTile), (unsigned)batch);
+    // 64 x 64 tiles for the cdist metrics and the power sums where 128 x 128 ones would leave CUs
+    // with less than two blocks (7/4 of the CUs: p = 3 breaks even at 0.97 of two blocks a CU, p = 1
+    // at two).  p = 1, 3001 x 1999 x 100 (384 tiles): 45 -> 34 us; p = 1.5, 928 x 46 x 76: 183 -> 44
+    constexpr bool kSmall = MODE == kRoot || MODE == kSum;
+    const bool small = kSmall && 4 * cdiv(m, kTile) * cdiv(n, kTile) * batch < 7 * (int64_t)device_cus() &&
+                       cdiv(n, 64) <= kMaxGridYZ;
+    const int64_t tile = small ? 64 : kTile;
+    dim3 grid((unsigned)cdiv(m, tile), (unsigned)cdiv(n, tile), (unsigned)batch);
     const bool vec = (d % 4 == 0) && aligned16(x1) && aligned16(x2) && aligned16(out) && aligned16(out16);
     const float pf = (float)p, inv_p = (float)(1.0 / p);
     const LaunchEvents ev = launch_events("lp_forward_kernel");
-    auto launch = [&](auto om) {
-        constexpr int OM = decltype(om)::value;
+    auto launch_tile = [&](auto om, auto tt) {
+        constexpr int OM = decltype(om)::value, TT = decltype(tt)::value;
         if (vec)
-            hipExtLaunchKernelGGL((lp_forward_kernel<MODE, PK, true, OM>), grid, dim3(kThreads), 0, s, ev.start,
+            hipExtLaunchKernelGGL((lp_forward_kernel<MODE, PK, true, OM, TT>), grid, dim3(kThreads), 0, s, ev.start,
                                   ev.stop, 0, x1, x2, w, n, m, d, pf, inv_p, out, post, rownum, out16);
         else
-            hipExtLaunchKernelGGL((lp_forward_kernel<MODE, PK, false, OM>), grid, dim3(kThreads), 0, s, ev.start,
+            hipExtLaunchKernelGGL((lp_forward_kernel<MODE, PK, false, OM, TT>), grid, dim3(kThreads), 0, s, ev.start,
                                   ev.stop, 0, x1, x2, w, n, m, d, pf, inv_p, out, post, rownum, out16);
+    };
+    auto launch = [&](auto om) {
+        if constexpr (kSmall) {
+            if (small) return launch_tile(om, std::integral_constant<int, 64>{});
+        }
+        launch_tile(om, std::integral_constant<int, kTile>{});
     };
     // the bf16 output exists for the cdist metrics (kRoot), the row-numerator divide for the
     // signal-to-noise ratio (kSum, p = 2), the exp for the laplacian (kRoot, p = 1) and rbf
@@ -1135,17 +1121,11 @@ int fill(float *p, int64_t len, float v, hipStream_t s) {
     return check_launch("fill_kernel");
 }
 
-// Blocks of the backward grid per CU that may be resident at once: the kernels use more
-// than 128 VGPRs (at most 4 waves per SIMD, i.e. 4 blocks of 4 waves per CU).
-constexpr int kMaxBlocksPerCU = 4;
+// Blocks of the backward grid per CU that the split count aims at: two, which every instance
+// fits at once.  A constant and not each instance's occupancy, so that two instances of one
+// backward (the exp-scaled gradient and the plain one) split and so round alike.
+constexpr int kSplitBlocksPerCU = 2;
 
-int device_cus() {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return 256;
-    return cus;
-}
 
 // Number of j splits for `slots` resident blocks: the (row block, feature block, batch)
 // grid alone fills base blocks; splitting j multiplies that, and a whole number of
@@ -1153,8 +1133,7 @@ int device_cus() {
 // stages, down to one: a block of few stages costs about 5 us a stage while its SIMDs hold one
 // wave each, so a small problem is as long as its longest split, and the partials of `slots`
 // blocks (32 or 64 KB each) take a few us to add (manhattan forward and backward 3001 x 1999 x
-// 100: 368 -> 200 us against splits of at least 512 pairs; 3176 x 3178 x 10: 328 -> 120).  More slots never give fewer splits, so the
-// workspace is sized with the largest slot count.
+// 100: 368 -> 200 us against splits of at least 512 pairs; 3176 x 3178 x 10: 328 -> 120).
 constexpr int64_t kMaxSplits = 64;
 int64_t lp_backward_splits(int64_t slots, int64_t batch, int64_t n, int64_t m, int64_t d, int64_t fw) {
     const int64_t base = cdiv(n, kBRows) * cdiv(d, fw) * batch;
@@ -1167,28 +1146,23 @@ int64_t lp_backward_splits(int64_t slots, int64_t batch, int64_t n, int64_t m, i
     const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
     return cdiv(m, jps);
 }
-int64_t max_slots() { return (int64_t)device_cus() * kMaxBlocksPerCU; }
+int64_t split_slots() { return (int64_t)device_cus() * kSplitBlocksPerCU; }
 
 // grad [batch, n, d] of the first operand (x2's gradient: pass x2 as x1, n <-> m, TR).
-template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW, bool EXPG = false>
+template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW, bool EXPG = false, bool WHOLE = false>
 int launch_backward(const float *g, const float *aux0, const float *aux1, const float *x1,
                     const float *x2, const float *w, int64_t batch, int64_t n, int64_t m, int64_t d,
                     double p, float *grad, float *part, hipStream_t s, const float *eo = nullptr,
                     float es = 0.0f, const uint32_t *gate = nullptr, uint32_t gate_run = 0,
                     int64_t *shared_splits = nullptr, bool finish = true) {
-    // the direct layout's staging lanes span two rows of m: their byte offsets are 32-bit
-    TPW_REQUIRE(TR || 4 * m + 128 < ((int64_t)1 << 32),
-                "backward: %lld columns exceed the kernel's 32-bit staging offsets", (long long)m);
-    auto kern = lp_backward_kernel<MODE, PK, TR, WGRAD, PRE, FW, EXPG>;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, 0) != hipSuccess || per_cu <= 0)
-        per_cu = 2;
-    if (per_cu > kMaxBlocksPerCU) per_cu = kMaxBlocksPerCU;
+    TPW_REQUIRE(TR || 4 * m + 128 < ((int64_t)1 << 32), "backward: %lld columns exceed the kernel's range",
+                (long long)m);
+    auto kern = lp_backward_kernel<MODE, PK, TR, WGRAD, PRE, FW, EXPG, WHOLE>;
     // gated instances of one backward share the first one's split count (and so the partials'
     // layout and the one sum_splits pass after the last)
     int64_t splits = shared_splits && *shared_splits > 0
                          ? *shared_splits
-                         : lp_backward_splits((int64_t)device_cus() * per_cu, batch, n, m, d, FW);
+                         : lp_backward_splits(split_slots(), batch, n, m, d, FW);
     if (shared_splits) *shared_splits = splits;
     const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
     dim3 grid((unsigned)cdiv(d, FW), (unsigned)cdiv(n, kBRows), (unsigned)(splits * batch));
@@ -1233,7 +1207,7 @@ struct BwdJob {
     uint32_t *flag = nullptr;  // a workspace word for the p = 1 range flag (nullptr: no wide p = 1)
 };
 
-template <int MODE, int PK, int FW, bool PRE, bool EXPG = false>
+template <int MODE, int PK, int FW, bool PRE, bool EXPG = false, bool WHOLE = false>
 int run_backward_fw(const BwdJob &j, hipStream_t s) {
     // staging reads the per-pair arrays only where the weights need them
     constexpr bool kAux = PRE || (MODE == kRoot && PK != kP1);
@@ -1249,14 +1223,14 @@ int run_backward_fw(const BwdJob &j, hipStream_t s) {
     int rc = TPW_OK;
     if (j.gx1) {
         if (j.x1_transposed)  // n, m are already those of the operand whose grad is wanted
-            rc = launch_backward<MODE, PK, true, false, PRE, FW, EXPG>(j.g, a0, a1, j.x1, j.x2, j.w, j.batch, j.n,
+            rc = launch_backward<MODE, PK, true, false, PRE, FW, EXPG, WHOLE>(j.g, a0, a1, j.x1, j.x2, j.w, j.batch, j.n,
                                                                     j.m, j.d, j.p, j.gx1, j.part, s, j.eo, j.es);
         else
-            rc = launch_backward<MODE, PK, false, false, PRE, FW, EXPG>(j.g, a0, a1, j.x1, j.x2, j.w, j.batch, j.n,
+            rc = launch_backward<MODE, PK, false, false, PRE, FW, EXPG, WHOLE>(j.g, a0, a1, j.x1, j.x2, j.w, j.batch, j.n,
                                                                      j.m, j.d, j.p, j.gx1, j.part, s, j.eo, j.es);
     }
     if (rc == TPW_OK && j.gx2)
-        rc = launch_backward<MODE, PK, true, false, PRE, FW, EXPG>(j.g, a0, a1, j.x2, j.x1, j.w, j.batch, j.m, j.n,
+        rc = launch_backward<MODE, PK, true, false, PRE, FW, EXPG, WHOLE>(j.g, a0, a1, j.x2, j.x1, j.w, j.batch, j.m, j.n,
                                                                 j.d, j.p, j.gx2, j.part, s, j.eo, j.es);
     if constexpr (MODE == kWeighted) {
         if (rc == TPW_OK && j.rows)
@@ -1270,7 +1244,7 @@ int run_backward_fw(const BwdJob &j, hipStream_t s) {
 // outside the pre-scaled sign path's range, then the wide kernel (sign path only; runs when the
 // flag is clear) and the narrow one (per-tile test and signf path; runs when it is set) are both
 // launched with the wide kernel's split count, and one sum_splits pass follows.
-template <int MODE, bool EXPG = false>
+template <int MODE, bool EXPG, bool WHOLE>
 int run_backward_p1_gated(const BwdJob &j, hipStream_t s) {
     int rc = fill(reinterpret_cast<float *>(j.flag), 1, 0.0f, s);
     if (rc != TPW_OK) return rc;
@@ -1283,7 +1257,7 @@ int run_backward_p1_gated(const BwdJob &j, hipStream_t s) {
     auto both = [&](auto tr, const float *xa, const float *xb, int64_t na, int64_t nb, float *grad) {
         constexpr bool TR = decltype(tr)::value;
         int64_t sp = 0;
-        int r = launch_backward<MODE, kP1, TR, false, false, kBFeatWide, EXPG>(
+        int r = launch_backward<MODE, kP1, TR, false, false, kBFeatWide, EXPG, WHOLE>(
             j.g, nullptr, nullptr, xa, xb, j.w, j.batch, na, nb, j.d, j.p, grad, j.part, s, j.eo, j.es, j.flag, 0u,
             &sp, false);
         if (r != TPW_OK) return r;
@@ -1300,23 +1274,25 @@ int run_backward_p1_gated(const BwdJob &j, hipStream_t s) {
     return rc;
 }
 
-// The wide kernel above 64 features where it serves the case and its 16-byte staging fits
-// (aligned arrays, n, m and d multiples of 4); else the narrow one.
-// Whether run_backward takes run_backward_p1_gated (p = 1: the wide kernel's shapes, and a flag word).
-bool p1_gated_fits(const BwdJob &j) {
-    return j.flag && j.d > kBFeat && j.n % 4 == 0 && j.m % 4 == 0 && j.d % 4 == 0 && aligned16(j.g) &&
-           aligned16(j.x1) && aligned16(j.x2) && aligned16(j.eo);
+// WHOLE's conditions (lp_backward_kernel): every array's row length a multiple of 4 and the
+// staging offsets of 128 rows below 2^32 bytes.  Any alignment: the loads need a dword's.
+bool whole_loads(const BwdJob &j) {
+    constexpr int64_t lim = ((int64_t)1 << 30) / kBRows - kBRows;
+    return j.n % 4 == 0 && j.m % 4 == 0 && j.d % 4 == 0 && j.n < lim && j.m < lim && j.d < lim;
 }
 
+// The wide kernel above 64 features where it serves the case, else the narrow one.
 template <int MODE, int PK, bool EXPG = false>
 int run_backward(const BwdJob &j, hipStream_t s) {
+    const bool whole = whole_loads(j);
     if constexpr (PK == kP1 && (MODE == kRoot || MODE == kSum)) {
-        if (p1_gated_fits(j)) return run_backward_p1_gated<MODE, EXPG>(j, s);
+        if (j.flag && j.d > kBFeat)
+            return whole ? run_backward_p1_gated<MODE, EXPG, true>(j, s) : run_backward_p1_gated<MODE, EXPG, false>(j, s);
     }
     if constexpr (kWide<MODE, PK>) {
-        const bool fits = j.d > kBFeat && j.n % 4 == 0 && j.m % 4 == 0 && j.d % 4 == 0 && aligned16(j.g) &&
-                          aligned16(j.aux0) && aligned16(j.x1) && aligned16(j.x2) && aligned16(j.eo);
-        if (fits) return run_backward_fw<MODE, PK, kBFeatWide, false, EXPG>(j, s);
+        if (j.d > kBFeat)
+            return whole ? run_backward_fw<MODE, PK, kBFeatWide, false, EXPG, true>(j, s)
+                         : run_backward_fw<MODE, PK, kBFeatWide, false, EXPG, false>(j, s);
     }
     static_assert(!EXPG || !kPrecomputed<MODE, PK>, "the exp-scaled gradient is formed while staging");
     return run_backward_fw<MODE, PK, kBFeat, kPrecomputed<MODE, PK>, EXPG>(j, s);
@@ -1351,7 +1327,7 @@ struct Workspace {
 };
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 Workspace workspace_layout(int metric, int64_t batch, int64_t n, int64_t m, int64_t d) {
-    const int64_t slots = max_slots();
+    const int64_t slots = split_slots();
     // the wide kernel's grid has fewer feature blocks, so it may take more splits
     int64_t s1 = lp_backward_splits(slots, batch, n, m, d, kBFeatWide);
     int64_t s2 = lp_backward_splits(slots, batch, m, n, d, kBFeatWide);
@@ -1694,8 +1670,8 @@ extern "C" int tpw_pairwise_exp_kernel_backward(const float *grad, const float *
                  nullptr, nullptr, false, out, -gamma};
         return run_backward<kSum, kP2, true>(j, s);
     }
-    // p = 1: on the wide kernel's shapes (run_backward_p1_gated) the gradient is formed while the
-    // kernels stage their pairs (the narrow fallback instance too, at two waves per SIMD: it runs
+    // p = 1: above 64 features (run_backward_p1_gated) the gradient is formed while the kernels
+    // stage their pairs (the narrow fallback instance too, at two waves per SIMD: it runs
     // only for values outside the sign path's range); elsewhere a second per-pair array would
     // take the narrow kernel from three waves per SIMD to two (156 -> 174 VGPRs), so one
     // elementwise pass writes the gradients into the workspace first
@@ -1703,7 +1679,7 @@ extern "C" int tpw_pairwise_exp_kernel_backward(const float *grad, const float *
         BwdJob j{grad, nullptr, nullptr, x1, x2, nullptr, batch, n, m, d, 1.0, grad_x1, grad_x2, nullptr, part,
                  nullptr, nullptr, false, out, -gamma};
         j.flag = lay.flag_word(ws);
-        if (p1_gated_fits(j)) return run_backward<kRoot, kP1, true>(j, s);
+        if (d > kBFeat) return run_backward<kRoot, kP1, true>(j, s);
     }
     const int64_t len = batch * n * m;
     const bool vec = aligned16(grad) && aligned16(out) && aligned16(pair1);
