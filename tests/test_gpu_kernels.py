@@ -552,6 +552,56 @@ def test_hausdorff_nonfinite_bit_exact(case):
     assert_equal(i2.cpu(), torch.from_numpy(w[2]), f"{case} idx2")
 
 
+# Small clouds on the dense kernels: blocks of 64 m (p1 = 63 .. 129), waves of 32 or more points of
+# x2 and eight a step (p2 = 1 .. 1025), permuted orders, duplicated points (the tie rules), and one
+# value that is not finite in one of the clouds
+@pytest.mark.parametrize("p1,p2", [(63, 1), (64, 31), (65, 33), (129, 255), (1, 513), (200, 1025), (700, 40)])
+@pytest.mark.parametrize("d", [1, 2, 3])
+@pytest.mark.parametrize("case", ["plain", "shuffled", "ties", "nan_x1", "inf_x2"])
+def test_hausdorff_dense_bit_exact(p1, p2, d, case):
+    x1, x2 = _hd_inputs(2, 2, p1, 3, p2, d, seed=50)
+    perm1 = perm2 = None
+    if case in ("shuffled", "ties"):
+        perm1, perm2 = P.hausdorff_permutations(2, p1, p2, torch.Generator().manual_seed(9))
+    if case == "ties":
+        x1, x2 = (x1 * 4).round() / 4, (x2 * 4).round() / 4
+    elif case == "nan_x1":
+        x1[1, 0, p1 // 2, d - 1] = float("nan")
+    elif case == "inf_x2":
+        x2[0, 2, p2 - 1, 0] = float("inf")
+    _hd_check(x1, x2, perm1, perm2, f"{case} {p1}x{p2}x{d}")
+
+
+def _hd_check(x1, x2, perm1, perm2, what):
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    host = lambda t: None if t is None else t.numpy()  # noqa: E731
+    got = capi.directed_hausdorff(x1.to(DEV), x2.to(DEV), dev(perm1), dev(perm2))
+    want = cref.directed_hausdorff(x1.numpy(), x2.numpy(), host(perm1), host(perm2), threads=8)
+    for g, w, nm in zip(got, want, ("value", "idx1", "idx2")):
+        assert_equal(g.cpu(), torch.from_numpy(w), f"{what} {nm}", nan_payload=False)
+
+
+# the grid's sorted mode at one pair of clouds past the dense kernels' 2^28 point pairs
+@pytest.mark.parametrize("case", ["offset", "flat", "shuffled", "ties", "self", "nan_x1"])
+def test_hausdorff_grid_above_dense_bit_exact(case):
+    x1, x2 = _hd_inputs(None, 1, 17000, 1, 16500, 3, seed=60)
+    perm1 = perm2 = None
+    if case == "offset":
+        x1, x2 = x1 + 1.0e4, x2 + 1.0e4
+    elif case == "flat":
+        x1[..., 2] = x2[..., 2] = 0.25
+    elif case == "shuffled":
+        perm1, perm2 = P.hausdorff_permutations(1, 17000, 16500, torch.Generator().manual_seed(11))
+    elif case == "ties":
+        x1, x2 = (x1 * 16).round() / 16, (x2 * 16).round() / 16
+    elif case == "self":
+        x2 = x1.clone()
+    else:
+        x1[0, 5, 1] = float("nan")
+        x1[0, 6:] = x1[0, 6:] * 0.1  # short early exits: the loop itself runs on one wave
+    _hd_check(x1, x2, perm1, perm2, case)
+
+
 def test_hausdorff_counters():
     """The work counters: the kernels evaluate far fewer pairs than brute force, the sorted
     mode's cell scan runs its box tests, the forward of a few clouds is ten launches, and
