@@ -78,6 +78,39 @@ def test_inner_tile_kernel_equals_staged_kernel(dtype, B, n, m, d, epi):
     assert _same_bits(tile, staged)
 
 
+# Small outputs (64 x 64 tiles, norms formed in the kernel or given) against the 128 x 128 kernels,
+# which the same rows take inside a batch of 260: the same products and norms in the same order, so
+# the same bits.  Tile edges, ragged m, rows of whole and partial 16-byte pieces, chunks (32 fp32,
+# 64 bf16) and 256-byte stages, vector norms of 1 .. 64 lanes, unaligned operands.  bf16 cosine
+# rounds its quotient by reciprocal norms where the whole tile allows it (2 ulp of float before the
+# bf16 rounding), and a tile with a zero row divides: one bf16 ulp between the two.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,m,d", [(64, 64, 64), (65, 63, 50), (1, 129, 1), (33, 100, 128), (130, 7, 257),
+                                   (40, 66, 100), (31, 32, 516)])
+@pytest.mark.parametrize("epi", EPIS)
+def test_small_output_kernel_equals_tile_kernels(dtype, n, m, d, epi):
+    B = 260
+    x1, x2 = randn(B, n, d, seed=21).to(DEV, dtype), randn(B, m, d, seed=22).to(DEV, dtype)
+    x2[:, min(3, m - 1)] = 0
+    def small(a, c, b):
+        return capi.lib().tpw_pairwise_inner_forms_norms(capi._ptr(a), capi._ptr(c), capi._dtype_code(a), b, n, m, d)
+
+    assert not small(x1, x2, B)
+    want = _inner(x1, x2, epi, False)
+    for b in (0, B - 1):
+        given = _inner(x1[b:b + 1].contiguous(), x2[b:b + 1].contiguous(), epi, b > 0)
+        own = torch.empty((1, n, m), dtype=dtype, device=DEV)
+        a, c = x1[b].clone(), x2[b].clone()
+        assert small(a, c, 1)
+        capi.call("tpw_pairwise_inner", capi._ptr(a), capi._ptr(c), capi._dtype_code(a), 1, n, m, d, None, None, epi,
+                  capi._ptr(own), capi._stream())
+        assert _same_bits(own, given)
+        if dtype == torch.bfloat16 and epi >= capi.EPI_COSINE_SIM:
+            assert torch.allclose(own[0].float(), want[b].float(), rtol=2.0 ** -7, atol=2.0 ** -8)
+        else:
+            assert _same_bits(own[0], want[b])
+
+
 def _fp4_metric(x1, x2, metric, misaligned):
     (fa, ca), (fb, cb) = capi.pack_bool_fp4(x1), capi.pack_bool_fp4(x2)
     B, n, d = x1.shape

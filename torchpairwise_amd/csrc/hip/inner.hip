@@ -22,6 +22,8 @@
 // Tiles are assigned XCD-contiguously (consecutive workgroup ids go round-robin over the
 // 8 XCDs, so id % 8 selects the XCD) and in groups of 8 tile rows, so that the blocks
 // resident on one XCD share A and B panels in that XCD's L2.
+#include <type_traits>
+
 #include "common.hpp"
 #include "tile_mfma.hpp"
 
@@ -711,6 +713,42 @@ __global__ __launch_bounds__(tile::kThreads, NB == 1 ? 4 : 2) void inner_tile_ke
     }
 }
 
+// The sum of squares of a row, by the lanes that share it, in the one order every norm uses (the
+// norm kernels and the small kernel's own norms agree bit for bit).  By element: 64 lanes, lane
+// `lane` taking k = lane, lane + 64, ...; by 16-byte vector: G lanes (a power of two), lane gl
+// taking vectors gl, gl + G, ...; then a butterfly over the lanes.
+template <typename T>
+__device__ __forceinline__ float row_sumsq(const T *__restrict__ p, int64_t d, int lane) {
+    float s = 0.0f;
+    for (int64_t k = lane; k < d; k += 64) {
+        float v;
+        if constexpr (sizeof(T) == 4) v = p[k];
+        else v = bf16_to_f32(p[k]);
+        s = __builtin_fmaf(v, v, s);
+    }
+    return s;
+}
+template <typename T>
+__device__ __forceinline__ float row_sumsq_vec(const uint4 *__restrict__ p, int64_t nv, int gl, int G) {
+    float s = 0.0f;
+    for (int64_t k = gl; k < nv; k += G) {
+        const uint4 v = p[k];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (sizeof(T) == 4) {
+                const float f = __uint_as_float(w[e]);
+                s = __builtin_fmaf(f, f, s);
+            } else {
+                const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xffff0000u);
+                s = __builtin_fmaf(lo, lo, s);
+                s = __builtin_fmaf(hi, hi, s);
+            }
+        }
+    }
+    return s;
+}
+
 // Row norms: one wave per row, lanes stride over the features.
 template <typename T>
 __global__ void row_norms_kernel(const T *__restrict__ x, int64_t rows, int64_t d, int squared,
@@ -718,14 +756,7 @@ __global__ void row_norms_kernel(const T *__restrict__ x, int64_t rows, int64_t 
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
-    const T *p = x + row * d;
-    float s = 0.0f;
-    for (int64_t k = lane; k < d; k += 64) {
-        float v;
-        if constexpr (sizeof(T) == 4) v = p[k];
-        else v = bf16_to_f32(p[k]);
-        s += v * v;
-    }
+    float s = row_sumsq(x + row * d, d, lane);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (lane == 0) out[row] = squared ? s : sqrt_rn(s);
@@ -742,41 +773,31 @@ __global__ __launch_bounds__(256) void row_norms_vec_kernel(const T *__restrict_
     const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / G) + lane / G;
     const int gl = lane % G;
     float s = 0.0f;
-    if (row < rows) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(x + row * d);
-        const int64_t nv = d / PER;
-        for (int64_t k = gl; k < nv; k += G) {
-            const uint4 v = p[k];
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if constexpr (sizeof(T) == 4) {
-                    const float f = __uint_as_float(w[e]);
-                    s += f * f;
-                } else {
-                    const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xffff0000u);
-                    s += lo * lo;
-                    s += hi * hi;
-                }
-            }
-        }
-    }
+    if (row < rows) s = row_sumsq_vec<T>(reinterpret_cast<const uint4 *>(x + row * d), d / PER, gl, G);
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (row < rows && gl == 0) out[row] = squared ? s : sqrt_rn(s);
 }
 
+// Lanes per row of the vector norms (the smallest power of two >= nv, at most 64), or 0 where
+// the rows are no whole aligned 16-byte vectors.
+template <typename T>
+int norm_lanes(const T *x, int64_t d) {
+    const int64_t nv = d * (int64_t)sizeof(T) / 16;
+    if ((d * (int64_t)sizeof(T)) % 16 != 0 || !aligned16(x) || nv == 0) return 0;
+    int g = 1;
+    while (g < 64 && g < nv) g *= 2;
+    return g;
+}
+
 template <typename T>
 int launch_row_norms(const T *x, int64_t rows, int64_t d, int squared, float *norms, hipStream_t s) {
-    const int64_t nv = d * (int64_t)sizeof(T) / 16;
-    if ((d * (int64_t)sizeof(T)) % 16 != 0 || !aligned16(x) || nv == 0) {
+    const int g = norm_lanes(x, d);
+    if (g == 0) {
         hipLaunchKernelGGL(row_norms_kernel<T>, dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, s, x, rows, d, squared,
                            norms);
         return check_launch("row_norms_kernel");
     }
-    // the smallest power of two >= nv (at most 64) lanes per row
-    int g = 1;
-    while (g < 64 && g < nv) g *= 2;
     const int64_t rows_per_block = 4 * (64 / g);
     const dim3 grid((unsigned)cdiv(rows, rows_per_block));
     switch (g) {
@@ -791,10 +812,265 @@ int launch_row_norms(const T *x, int64_t rows, int64_t d, int squared, float *no
     return check_launch("row_norms_vec_kernel");
 }
 
+// ---------------------------------------------------------------------------------------
+// Small outputs: 64 x 64 tiles, four waves of one 32 x 32 block each, any d, m and alignment.  A
+// grid of 128 x 128 tiles that leaves most CUs without a block is as long as one tile: two or
+// three launches of 10 to 20 us for outputs that take the arithmetic of a microsecond.  A quarter
+// of the tile is a quarter of the chain, on four times the CUs, and with NORMS the block forms
+// the norms of its own 64 + 64 rows (in the norm kernels' order: same bits), so that the call is
+// one launch.  A stage is 256 bytes of every row (two K chunks of the tile kernel, multiplied in
+// the same order: same bits), the next stage's loads in flight meanwhile, 16 bytes at any element
+// alignment.  The MFMA's lanes hold neighbouring columns, so a dword store covers 128 contiguous
+// bytes of two rows at any m.
+constexpr int kST = 64;             // tile rows and columns
+constexpr int kSPieces = 16;        // 16-byte pieces per row and stage
+constexpr int kSStride = kSPieces + 1;
+
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
+
+// Piece of row r at element k, any element alignment, zero past d or the last row.
+template <typename T>
+__device__ __forceinline__ uint4 load_piece_any(const T *__restrict__ x, int64_t rows, int64_t d, int64_t r,
+                                                int64_t k) {
+    constexpr int E = Elem<T>::kPer16;
+    uint4 v = {0u, 0u, 0u, 0u};
+    if (r >= rows || k >= d) return v;
+    if (k + E <= d) {
+        if constexpr (E == 4) {
+            const floatx4u t = *reinterpret_cast<const floatx4u *>(x + r * d + k);
+            v = make_uint4(__float_as_uint(t[0]), __float_as_uint(t[1]), __float_as_uint(t[2]), __float_as_uint(t[3]));
+        } else {
+            const u32x4u t = *reinterpret_cast<const u32x4u *>(x + r * d + k);
+            v = make_uint4(t[0], t[1], t[2], t[3]);
+        }
+        return v;
+    }
+    return load_piece<T, false>(x, rows, d, r, k);
+}
+
+// The square sums of one row's share of a thread (its pieces c and c + 8 of every stage, eight
+// threads a row) in the order of row_sumsq / row_sumsq_vec, whose 64 lanes are here eight partial
+// sums in each of eight threads:
+//   vectors: lane = vector % 64 is thread c's sum 2 stage + half (mod 8).  The sums rotate by two
+//     each stage, so that the index is static; the butterfly's pairs (lanes 32, 16 and 8 apart)
+//     are four, two and one sums apart under any rotation;
+//   elements, fp32: lane = 32 half + 4 c + i, bf16: lane = 8 c + i, element i of the piece.
+// A lane without a value of its own adds zero, which changes no sum of squares.
+template <typename T>
+struct RowSquares {
+    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    static __device__ __forceinline__ float elem(const uint32_t (&w)[4], int i) {
+        if constexpr (sizeof(T) == 4) return __uint_as_float(w[i]);
+        else return __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
+    }
+    __device__ __forceinline__ void add(const uint4 &p0, const uint4 &p1, bool vec) {
+        constexpr int E = 16 / (int)sizeof(T);
+        const uint32_t w[2][4] = {{p0.x, p0.y, p0.z, p0.w}, {p1.x, p1.y, p1.z, p1.w}};
+        if (vec) {
+            float t[2] = {s[0], s[1]};
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+                for (int i = 0; i < E; ++i) t[hh] = __builtin_fmaf(elem(w[hh], i), elem(w[hh], i), t[hh]);
+#pragma unroll
+            for (int j = 0; j < 6; ++j) s[j] = s[j + 2];
+            s[6] = t[0];
+            s[7] = t[1];
+        } else {
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const int j = E == 4 ? 4 * hh + i : i;
+                    s[j] = __builtin_fmaf(elem(w[hh], i), elem(w[hh], i), s[j]);
+                }
+        }
+    }
+    // the row's sum, in each of its eight threads (tid % 8 = c)
+    __device__ __forceinline__ float total(bool vec) {
+        auto across = [](float v, int off) { return v + __shfl_xor(v, off, 64); };
+        auto local = [&](int off) {  // butterfly over the sums
+#pragma unroll
+            for (int j = 0; j < off; ++j) s[j] += s[j + off];
+        };
+        if (vec) {  // 32, 16, 8, then 4, 2, 1
+            local(4), local(2), local(1);
+            return across(across(across(s[0], 4), 2), 1);
+        }
+        if constexpr (sizeof(T) == 4) local(4);  // lanes 32 apart
+        constexpr int N = sizeof(T) == 4 ? 4 : 8;
+#pragma unroll
+        for (int j = 0; j < N; ++j) s[j] = across(across(across(s[j], 4), 2), 1);
+        if constexpr (sizeof(T) == 2) local(4);
+        local(2), local(1);
+        return s[0];
+    }
+};
+
+template <typename T, int EPI, bool NORMS>
+__global__ __launch_bounds__(kThreads) void inner_small_kernel(
+    const T *__restrict__ x1, const T *__restrict__ x2, int64_t n, int64_t m, int64_t d, bool vec1, bool vec2,
+    const float *__restrict__ aux1, const float *__restrict__ aux2, T *__restrict__ out, int64_t tiles_n,
+    int64_t tiles_m, int64_t total) {
+    __shared__ uint4 panels[2][kST * kSStride];
+    __shared__ float s_aux[2 * kST];  // norms of the tile's rows, then its columns
+    constexpr int E = Elem<T>::kPer16;
+    constexpr bool kOwn = kAux1<EPI> && NORMS;
+    int64_t b, tr, tc;
+    xcd_tile_of(blockIdx.x, tiles_n, tiles_m, total, b, tr, tc);
+    const int64_t row0 = tr * kST, col0 = tc * kST;
+    const T *A = x1 + b * n * d, *B = x2 + b * m * d;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+    const int l32 = lane & 31, h = lane >> 5;
+
+    // piece q of the thread and operand: row (tid >> 3) + 32 (q >> 1), piece (tid & 7) + 8 (q & 1)
+    constexpr int Q = kST * kSPieces / kThreads;
+    static_assert(Q == 4, "two rows of two pieces");
+    const int pr = tid >> 3, pc = tid & 7;
+    uint4 pa[Q], pb[Q];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int r = pr + 32 * (q >> 1);
+            const int64_t k = k0 + (int64_t)(pc + 8 * (q & 1)) * E;
+            pa[q] = load_piece_any<T>(A, n, d, row0 + r, k);
+            pb[q] = load_piece_any<T>(B, m, d, col0 + r, k);
+        }
+    };
+    load(0);
+    RowSquares<T> sq[kOwn ? 4 : 1];  // the thread's rows pr, pr + 32 of x1, then of x2
+    if constexpr (kAux1<EPI> && !NORMS) {
+        if (tid < kST) s_aux[tid] = row0 + tid < n ? aux1[b * n + row0 + tid] : 0.0f;
+        else if (tid < 2 * kST) s_aux[tid] = col0 + tid - kST < m ? aux2[b * m + col0 + tid - kST] : 0.0f;
+    }
+
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    constexpr int64_t KS = kSPieces * E;  // features per stage
+    for (int64_t k0 = 0; k0 < d; k0 += KS) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int at = (pr + 32 * (q >> 1)) * kSStride + pc + 8 * (q & 1);
+            panels[0][at] = pa[q];
+            panels[1][at] = pb[q];
+        }
+        if constexpr (kOwn) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                sq[u].add(pa[2 * u], pa[2 * u + 1], vec1);
+                sq[2 + u].add(pb[2 * u], pb[2 * u + 1], vec2);
+            }
+        }
+        __syncthreads();
+        if (k0 + KS < d) load(k0 + KS);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (k0 + half * (KS / 2) >= d) break;  // no features in the second chunk
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint4 a = panels[0][(wr + l32) * kSStride + 8 * half + 4 * h + q];
+                const uint4 c = panels[1][(wc + l32) * kSStride + 8 * half + 4 * h + q];
+                if constexpr (E == 4) {
+                    const uint32_t av[4] = {a.x, a.y, a.z, a.w}, cv[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(av[e]), __uint_as_float(cv[e]), acc,
+                                                                   0, 0, 0);
+                } else {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                                  __builtin_bit_cast(bf16x8, c), acc, 0, 0, 0);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if constexpr (kOwn) {
+        constexpr bool squared = EPI == TPW_EPI_EUCLIDEAN || EPI == TPW_EPI_SQEUCLIDEAN;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float t = sq[u].total(u < 2 ? vec1 : vec2);
+            if (pc == 0) s_aux[32 * u + pr] = squared ? t : sqrt_rn(t);
+        }
+    }
+    if (kOwn || d == 0) __syncthreads();  // the norms
+
+    bool rcp = false;  // bf16 cosine family: reciprocal norms where every norm of the tile allows it
+    if constexpr (kCosRcp<EPI, T>) {
+        const float v = tid < 2 * kST ? s_aux[tid] : 1.0f;
+        // rows and columns past the edge hold norm 0, which no output reads
+        const bool edge = tid < kST ? row0 + tid >= n : tid < 2 * kST ? col0 + tid - kST >= m : true;
+        rcp = __syncthreads_and(edge || (v >= 0x1p-60f && v <= 0x1p60f)) != 0;
+        if (rcp && tid < 2 * kST) s_aux[tid] = __fdiv_rn(1.0f, v);
+        __syncthreads();
+    }
+    // accumulator register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
+    const int64_t col = col0 + wc + l32;
+    if (col >= m) return;
+    const float a2 = kAux2<EPI> ? s_aux[kST + wc + l32] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int rr = wr + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (row0 + rr >= n) continue;
+        const float a1 = kAux1<EPI> ? s_aux[rr] : 0.0f;
+        float v;
+        if constexpr (kCosRcp<EPI, T>) v = rcp ? cos_epilogue_rcp<EPI>(acc[r], a1, a2) : epilogue<EPI>(acc[r], a1, a2, {});
+        else v = epilogue<EPI>(acc[r], a1, a2, {});
+        from_f32(out + (b * n + row0 + rr) * m + col, v);
+    }
+}
+
+// Compute units of the current device (256 when the query fails), per device.
+int64_t cu_count() {
+    static int cache[16];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+    int &c = cache[dev & 15];
+    if (c == 0) {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            cus = 256;
+        c = cus;
+    }
+    return c;
+}
+
+// Whether the small kernel takes the call: up to half as many 128 x 128 tiles as CUs, or as many
+// where the tile kernel would need padded copies of the operands or the staged kernel would run
+// (rows that are no whole aligned chunks, fp32 rows of m % 4 != 0 outputs).  Whole call, norms
+// launched -> formed inside: fp32 37 x 1003 x 50 15.3 -> 6.8 us, 700 x 900 x 128 17.5 -> 8.9, 8 x
+// 227 x 544 x 224 26.7 -> 16.8; bf16 1501 x 999 x 100 34.8 -> 10.2; at 144 tiles of d = 512 42.6
+// -> 41.9; at 256 tiles of whole chunks the tile kernel stays ahead (2048^2: d = 128 20.2 against
+// 23.1, d = 512 43.4 against 69.4), ragged 2047 x 2041 x 101 34.9 -> 23.8.
+template <typename T>
+bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d) {
+    const bool whole = d % Elem<T>::kChunk == 0 && aligned16(x1) && aligned16(x2) && (sizeof(T) == 2 || m % 4 == 0);
+    return cdiv(n, kTile) * cdiv(m, kTile) * batch * (whole ? 2 : 1) <= cu_count();
+}
+
+template <typename T, int EPI>
+int launch_small(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d, const float *aux1,
+                 const float *aux2, T *out, hipStream_t s) {
+    const int64_t tiles_n = cdiv(n, kST), tiles_m = cdiv(m, kST), total = tiles_n * tiles_m * batch;
+    const LaunchEvents ev = launch_events("inner_small_kernel");
+    if (kAux1<EPI> && !aux1)
+        hipExtLaunchKernelGGL((inner_small_kernel<T, EPI, true>), dim3((unsigned)total), dim3(kThreads), 0, s, ev.start,
+                              ev.stop, 0, x1, x2, n, m, d, norm_lanes(x1, d) != 0, norm_lanes(x2, d) != 0, aux1, aux2, out,
+                              tiles_n, tiles_m, total);
+    else
+        hipExtLaunchKernelGGL((inner_small_kernel<T, EPI, false>), dim3((unsigned)total), dim3(kThreads), 0, s,
+                              ev.start, ev.stop, 0, x1, x2, n, m, d, false, false, aux1, aux2, out, tiles_n, tiles_m, total);
+    return check_launch("inner_small_kernel");
+}
+
 template <typename T, int EPI, typename OutT = T>
 int launch_inner(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d,
                  const float *aux1, const float *aux2, OutT *out, hipStream_t s,
                  const OutT *X = nullptr, float sign = 1.0f, KerParams kp = {}) {
+    if constexpr (EPI <= TPW_EPI_CORRELATION && std::is_same<T, OutT>::value) {
+        if (small_fits(x1, x2, batch, n, m, d)) return launch_small<T, EPI>(x1, x2, batch, n, m, d, aux1, aux2, out, s);
+    }
     const int64_t tiles_n = cdiv(n, kTile), tiles_m = cdiv(m, kTile);
     const int64_t total = tiles_n * tiles_m * batch;
     const bool vec = ((d * (int64_t)sizeof(T)) % 16 == 0) && aligned16(x1) && aligned16(x2);
@@ -999,21 +1275,6 @@ int launch_grad_product(const T *A, const T *B, int64_t batch, int64_t M, int64_
     return check_launch("inner_tile_kernel");
 }
 
-// Compute units of the current device (256 when the query fails), per device.
-static int64_t cu_count() {
-    static int cache[16];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
-    int &c = cache[dev & 15];
-    if (c == 0) {
-        int cus = 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-        c = cus;
-    }
-    return c;
-}
-
 // The bf16 gradient product of launch_grad_product (out = sign * A'B + coef[row] * X, kEpiGrad,
 // or with coef the row sums of A, kEpiGradA) for both operands k-major (A: [K, M], B: [K, N])
 // on 128 x 256 output tiles, 2 x 2 waves of 64 x 128.  Each wave feeds eight 32x32x16 products
@@ -1195,6 +1456,16 @@ extern "C" int tpw_row_norms(const void *x, int dtype, int64_t rows, int64_t d, 
     return launch_row_norms(static_cast<const uint16_t *>(x), rows, d, squared, norms, s);
 }
 
+extern "C" int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
+                                              int64_t m, int64_t d) {
+    if (batch < 0 || n < 0 || m < 0 || d < 0 || (dtype != TPW_F32 && dtype != TPW_BF16)) return 0;
+    return (dtype == TPW_F32
+                ? small_fits(static_cast<const float *>(x1), static_cast<const float *>(x2), batch, n, m, d)
+                : small_fits(static_cast<const uint16_t *>(x1), static_cast<const uint16_t *>(x2), batch, n, m, d))
+               ? 1
+               : 0;
+}
+
 extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch,
                                   int64_t n, int64_t m, int64_t d, const float *aux1,
                                   const float *aux2, int epilogue, void *out, void *stream) {
@@ -1204,8 +1475,9 @@ extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int
     TPW_REQUIRE(batch >= 0 && n >= 0 && m >= 0 && d >= 0, "invalid sizes");
     if (batch == 0 || n == 0 || m == 0) return TPW_OK;
     TPW_REQUIRE(x1 && x2 && out, "null pointer");
-    TPW_REQUIRE(epilogue == TPW_EPI_DOT || (aux1 && aux2), "norms required for epilogue %d",
-                epilogue);
+    TPW_REQUIRE(epilogue == TPW_EPI_DOT || (aux1 && aux2) ||
+                    (!aux1 && !aux2 && tpw_pairwise_inner_forms_norms(x1, x2, dtype, batch, n, m, d)),
+                "norms required for epilogue %d", epilogue);
     const int64_t total = cdiv(n, kTile) * cdiv(m, kTile) * batch;
     TPW_REQUIRE(total <= 0x7fffffffLL, "output too large for one launch");
     hipStream_t s = as_stream(stream);

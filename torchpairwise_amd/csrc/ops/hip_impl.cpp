@@ -93,7 +93,9 @@ at::Tensor pw_inner_cuda(const at::Tensor &x1, const at::Tensor &x2, int64_t epi
     auto out = at::empty({B, n, m}, a.options());
     at::Tensor n1, n2;
     void *s = current_stream();
-    if (epilogue != TPW_EPI_DOT) {
+    // small outputs: one launch, norms inside
+    const bool small = tpw_pairwise_inner_forms_norms(a.data_ptr(), b.data_ptr(), dt, B, n, m, d) != 0;
+    if (epilogue != TPW_EPI_DOT && !small) {
         const int squared = (epilogue == TPW_EPI_EUCLIDEAN || epilogue == TPW_EPI_SQEUCLIDEAN);
         n1 = at::empty({B, n}, a.options().dtype(at::kFloat));
         check_rc(tpw_row_norms(a.data_ptr(), dt, B * n, d, squared, n1.data_ptr<float>(), s), "row norms");
@@ -107,12 +109,13 @@ at::Tensor pw_inner_cuda(const at::Tensor &x1, const at::Tensor &x2, int64_t epi
     // Rows that are not whole 128-byte chunks (or operands not 16-byte aligned) would take the
     // register-staged kernel, whose element loads run 1.3-4x slower; for outputs of 2^20 entries
     // or more the operands are copied zero-padded to whole chunks for the tile kernel instead.
-    // The staged kernel zero-fills its last chunk the same way, so the products are the same.
+    // The staged kernel zero-fills its last chunk the same way, so the products are the same.  (The
+    // small-output kernel loads any row.)
     at::Tensor ap = a, bp = b;
     int64_t dk = d;
     const int64_t chunk = 128 / (int64_t)a.element_size();
     const auto misaligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
-    if (d > 0 && B * n * m >= (int64_t(1) << 20) &&
+    if (!small && d > 0 && B * n * m >= (int64_t(1) << 20) &&
         (d % chunk != 0 || misaligned(a.data_ptr()) || misaligned(b.data_ptr()))) {
         dk = (d + chunk - 1) / chunk * chunk;
         ap = at::zeros({B, n, dk}, a.options());
