@@ -307,6 +307,11 @@ int tpw_compare_reduce(const void *x1, const void *x2, int elem_type, int64_t ba
 int tpw_row_norms(const void *x, int dtype, int64_t rows, int64_t d, int squared,
                   float *norms, void *stream);
 
+/* tpw_row_norms of two operands of equal d in one launch (same bits): the same two reference
+ * reductions. */
+int tpw_row_norms2(const void *x1, int64_t rows1, const void *x2, int64_t rows2, int dtype,
+                   int64_t d, int squared, float *norms1, float *norms2, void *stream);
+
 /* out[b,i,j] = epilogue(x1[b,i,:] . x2[b,j,:], aux1[b*n+i], aux2[b*m+j]) with the
  * contraction on the matrix cores (fp32: v_mfma_f32_32x32x2_f32; bf16:
  * v_mfma_f32_32x32x16_bf16, fp32 accumulation).  aux1/aux2 are the squared norms

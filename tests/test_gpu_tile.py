@@ -234,6 +234,85 @@ def test_backward_products_tile_fp32(name, kw, B, n, m, d):
         assert_close(tile, split.double(), rtol=0, atol=1e-5 * scale, what=f"{name} grad_x{k + 1} tile vs split-K")
 
 
+# Both gradients in one launch (op_backward_kernel): edges of its 64-row tiles, 64- and 128-feature
+# tiles, 32-row K chunks and splits, sums long enough to be blocked (512), vector and element
+# loads; a zero row (norm 0) and rows out of the fast cosine terms' norm range.  fp32 against the
+# derived per-element bounds (euclidean, cosine) or, like the kernel functions above, rtol 1e-4;
+# bf16 at the bf16 tolerance of the other paths.
+@pytest.mark.parametrize("B,n,m,d", [(1, 1, 1, 1), (1, 63, 65, 64), (2, 65, 33, 65), (1, 31, 1100, 30),
+                                     (1, 1601, 64, 128), (3, 130, 97, 131)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name,kw", [o for o in BWD_OPS if o[0] != "polynomial_kernel"])
+def test_backward_one_launch(name, kw, dtype, B, n, m, d):
+    import torchpairwise_amd as tp
+    from tests import _gradbound as GB
+    from tests._util import assert_close
+
+    print(f"one launch {name} {dtype} B={B} n={n} m={m} d={d}", flush=True)
+    fn = getattr(tp, name)
+    x1, x2, g = (randn(B, r, c, seed=k, dtype=dtype) for k, (r, c) in enumerate(((n, d), (m, d), (n, m))))
+    if n > 40 and name.startswith("cosine"):
+        x1[:, 7] = 0
+        x1[:, 33] *= 2.0 ** 58  # norm about 2^61
+    a, b = x1.to(DEV).requires_grad_(), x2.to(DEV).requires_grad_()
+    fn(a, b, **kw).backward(g.to(DEV))
+    ra, rb = x1.double().requires_grad_(), x2.double().requires_grad_()
+    fn(ra, rb, **kw).backward(g.double())
+    plain = slice(34, None) if n > 40 and name.startswith("cosine") else slice(None)
+    for k, (got, want) in enumerate(((a.grad, ra.grad), (b.grad, rb.grad))):
+        if dtype == torch.float32 and name in ("euclidean_distances", "cosine_similarity") and d > 1:
+            for bb in range(B):
+                own, other, gs = (x1, x2, g[bb]) if k == 0 else (x2, x1, g[bb].T)
+                if name == "euclidean_distances":
+                    bound = GB.euclidean_grad_bound(own[bb], other[bb], gs)
+                elif k == 0:  # rows of ordinary norms
+                    GB.check(got[bb].cpu()[plain], want[bb][plain],
+                             GB.cosine_grad_bound(own[bb], other[bb], gs, True)[plain], f"{name} grad_x1")
+                    continue
+                else:
+                    ok = torch.ones(n, dtype=torch.bool)
+                    if n > 40:
+                        ok[7] = False  # the zero row's pairs: no quotient
+                    bound = GB.cosine_grad_bound(own[bb], other[bb][ok], gs[:, ok], True)
+                GB.check(got[bb].cpu(), want[bb], bound, f"{name} grad_x{k + 1}")
+        tol = 1e-4 if dtype == torch.float32 else 1e-2
+        # one feature: the cosine's two terms, each at most |g| / |own| a pair, cancel to zero, and
+        # what is left is their rounding (4 u a term, u = 2^-24 or 2^-9)
+        own = (x1, x2)[k].double()
+        left = 0.0
+        if d == 1:
+            u = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -9
+            left = 4 * u * float(g.double().abs().sum()) / max(float(own.abs().min()), 1e-3)
+        # (the row scaled by 2^58 has gradients 2^-58 of the others': the floor covers them)
+        assert_close(got.float(), want, rtol=tol, atol=tol * float(want.abs().max()) + left,
+                     what=f"{name} grad_x{k + 1}")
+
+
+# past op_backward_kernel's limit (3 2^23 pairs): the weight pass and the products, fp32 split-K
+# and tile kernel and bf16 with W^T and transposed copies, ragged and aligned, against float64 on
+# the GPU's plain torch operations
+@pytest.mark.parametrize("n,m,d", [(5201, 5003, 70), (5120, 5120, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name", ["euclidean_distances", "cosine_similarity", "linear_kernel"])
+def test_backward_passes_above_one_launch(name, dtype, n, m, d):
+    import torchpairwise_amd as tp
+    from tests._util import assert_close
+
+    x1, x2, g = randn(n, d, seed=0, dtype=dtype), randn(m, d, seed=1, dtype=dtype), randn(n, m, seed=2, dtype=dtype)
+    a, b, gd = x1.to(DEV).requires_grad_(), x2.to(DEV).requires_grad_(), g.to(DEV)
+    getattr(tp, name)(a, b).backward(gd)
+    ra, rb = (x.to(DEV).double().requires_grad_() for x in (x1, x2))
+    s = ra @ rb.T
+    if name == "euclidean_distances":
+        s = (ra.square().sum(1)[:, None] + rb.square().sum(1)[None] - 2 * s).clamp_min(0).sqrt()
+    elif name == "cosine_similarity":
+        s = s / (ra.norm(dim=1)[:, None] * rb.norm(dim=1)[None])
+    s.backward(gd.double())
+    tol = 1e-4 if dtype == torch.float32 else 1e-2
+    for got, want in ((a.grad, ra.grad), (b.grad, rb.grad)):
+        assert_close(got.float(), want, rtol=tol, atol=tol * float(want.abs().max()), what=name)
+
+
 # bf16: x2 (for grad_x1) and W, x1 (for grad_x2) read k-major through transposing LDS reads,
 # and (euclidean, sigmoid; n % 128 == 0) the weights formed inside the grad_x1 product, against
 # the path that inputs offset by one element take (W^T and transposed copies of x1, x2

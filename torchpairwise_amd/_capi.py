@@ -47,6 +47,7 @@ _SIGNATURES = {
     "tpw_count_division_check": (_i, [_i64, _i64, _i64, _i64, _p, _p]),
     "tpw_compare_reduce": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _i, _i, _p, _p]),
     "tpw_row_norms": (_i, [_p, _i, _i64, _i64, _i, _p, _p]),
+    "tpw_row_norms2": (_i, [_p, _i64, _p, _i64, _i, _i64, _i, _p, _p, _p]),
     "tpw_pairwise_inner": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _p, _p, _i, _p, _p]),
     "tpw_pairwise_inner_forms_norms": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64]),
     "tpw_radius_mask_euclidean": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _p, _p, C.c_float, _p, _p]),

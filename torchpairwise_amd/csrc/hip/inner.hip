@@ -749,34 +749,47 @@ __device__ __forceinline__ float row_sumsq_vec(const uint4 *__restrict__ p, int6
     return s;
 }
 
+// The rows of one or two operands, those of the second after those of the first.
+template <typename T>
+struct NormRows {
+    const T *x1, *x2;
+    float *out1, *out2;
+    int64_t rows1, rows;
+    __device__ __forceinline__ const T *row(int64_t r, int64_t d) const {
+        return r < rows1 ? x1 + r * d : x2 + (r - rows1) * d;
+    }
+    __device__ __forceinline__ void put(int64_t r, float v) const {
+        if (r < rows1) out1[r] = v;
+        else out2[r - rows1] = v;
+    }
+};
+
 // Row norms: one wave per row, lanes stride over the features.
 template <typename T>
-__global__ void row_norms_kernel(const T *__restrict__ x, int64_t rows, int64_t d, int squared,
-                                 float *__restrict__ out) {
+__global__ void row_norms_kernel(NormRows<T> x, int64_t d, int squared) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (row >= rows) return;
-    float s = row_sumsq(x + row * d, d, lane);
+    if (row >= x.rows) return;
+    float s = row_sumsq(x.row(row, d), d, lane);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) out[row] = squared ? s : sqrt_rn(s);
+    if (lane == 0) x.put(row, squared ? s : sqrt_rn(s));
 }
 
 // Row norms with 16-byte loads (rows of whole 16-byte vectors, 16-byte aligned): G lanes per
 // row (a power of two, G >= the row's vector count up to 64), 64 / G rows per wave; each lane
 // sums the squares of its vectors, then a butterfly over the G lanes.
 template <typename T, int G>
-__global__ __launch_bounds__(256) void row_norms_vec_kernel(const T *__restrict__ x, int64_t rows, int64_t d,
-                                                            int squared, float *__restrict__ out) {
+__global__ __launch_bounds__(256) void row_norms_vec_kernel(NormRows<T> x, int64_t d, int squared) {
     constexpr int PER = 16 / (int)sizeof(T);
     const int lane = threadIdx.x & 63;
     const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / G) + lane / G;
     const int gl = lane % G;
     float s = 0.0f;
-    if (row < rows) s = row_sumsq_vec<T>(reinterpret_cast<const uint4 *>(x + row * d), d / PER, gl, G);
+    if (row < x.rows) s = row_sumsq_vec<T>(reinterpret_cast<const uint4 *>(x.row(row, d)), d / PER, gl, G);
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (row < rows && gl == 0) out[row] = squared ? s : sqrt_rn(s);
+    if (row < x.rows && gl == 0) x.put(row, squared ? s : sqrt_rn(s));
 }
 
 // Lanes per row of the vector norms (the smallest power of two >= nv, at most 64), or 0 where
@@ -791,23 +804,23 @@ int norm_lanes(const T *x, int64_t d) {
 }
 
 template <typename T>
-int launch_row_norms(const T *x, int64_t rows, int64_t d, int squared, float *norms, hipStream_t s) {
-    const int g = norm_lanes(x, d);
+int launch_row_norms(const NormRows<T> &x, int64_t d, int squared, hipStream_t s) {
+    const int g = norm_lanes(x.x1, d);
+    const int64_t rows = x.rows;
     if (g == 0) {
-        hipLaunchKernelGGL(row_norms_kernel<T>, dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, s, x, rows, d, squared,
-                           norms);
+        hipLaunchKernelGGL(row_norms_kernel<T>, dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, s, x, d, squared);
         return check_launch("row_norms_kernel");
     }
     const int64_t rows_per_block = 4 * (64 / g);
     const dim3 grid((unsigned)cdiv(rows, rows_per_block));
     switch (g) {
-        case 1: hipLaunchKernelGGL((row_norms_vec_kernel<T, 1>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        case 2: hipLaunchKernelGGL((row_norms_vec_kernel<T, 2>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        case 4: hipLaunchKernelGGL((row_norms_vec_kernel<T, 4>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        case 8: hipLaunchKernelGGL((row_norms_vec_kernel<T, 8>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        case 16: hipLaunchKernelGGL((row_norms_vec_kernel<T, 16>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        case 32: hipLaunchKernelGGL((row_norms_vec_kernel<T, 32>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
-        default: hipLaunchKernelGGL((row_norms_vec_kernel<T, 64>), grid, dim3(256), 0, s, x, rows, d, squared, norms); break;
+        case 1: hipLaunchKernelGGL((row_norms_vec_kernel<T, 1>), grid, dim3(256), 0, s, x, d, squared); break;
+        case 2: hipLaunchKernelGGL((row_norms_vec_kernel<T, 2>), grid, dim3(256), 0, s, x, d, squared); break;
+        case 4: hipLaunchKernelGGL((row_norms_vec_kernel<T, 4>), grid, dim3(256), 0, s, x, d, squared); break;
+        case 8: hipLaunchKernelGGL((row_norms_vec_kernel<T, 8>), grid, dim3(256), 0, s, x, d, squared); break;
+        case 16: hipLaunchKernelGGL((row_norms_vec_kernel<T, 16>), grid, dim3(256), 0, s, x, d, squared); break;
+        case 32: hipLaunchKernelGGL((row_norms_vec_kernel<T, 32>), grid, dim3(256), 0, s, x, d, squared); break;
+        default: hipLaunchKernelGGL((row_norms_vec_kernel<T, 64>), grid, dim3(256), 0, s, x, d, squared); break;
     }
     return check_launch("row_norms_vec_kernel");
 }
@@ -1452,8 +1465,32 @@ extern "C" int tpw_row_norms(const void *x, int dtype, int64_t rows, int64_t d, 
     if (rows == 0) return TPW_OK;
     TPW_REQUIRE(x && norms, "null pointer");
     hipStream_t s = as_stream(stream);
-    if (dtype == TPW_F32) return launch_row_norms(static_cast<const float *>(x), rows, d, squared, norms, s);
-    return launch_row_norms(static_cast<const uint16_t *>(x), rows, d, squared, norms, s);
+    if (dtype == TPW_F32) {
+        const float *p = static_cast<const float *>(x);
+        return launch_row_norms(NormRows<float>{p, p, norms, norms, rows, rows}, d, squared, s);
+    }
+    const uint16_t *p = static_cast<const uint16_t *>(x);
+    return launch_row_norms(NormRows<uint16_t>{p, p, norms, norms, rows, rows}, d, squared, s);
+}
+
+extern "C" int tpw_row_norms2(const void *x1, int64_t rows1, const void *x2, int64_t rows2, int dtype, int64_t d,
+                              int squared, float *norms1, float *norms2, void *stream) {
+    // one launch where both operands take the same kernel, the same bits as two
+    auto run = [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        const T *a = static_cast<const T *>(x1), *b = static_cast<const T *>(x2);
+        if (norm_lanes(a, d) == norm_lanes(b, d))
+            return launch_row_norms(NormRows<T>{a, b, norms1, norms2, rows1, rows1 + rows2}, d, squared,
+                                    as_stream(stream));
+        const int rc = tpw_row_norms(x1, dtype, rows1, d, squared, norms1, stream);
+        return rc != TPW_OK ? rc : tpw_row_norms(x2, dtype, rows2, d, squared, norms2, stream);
+    };
+    TPW_REQUIRE(dtype == TPW_F32 || dtype == TPW_BF16, "unsupported dtype %d", dtype);
+    TPW_REQUIRE(rows1 >= 0 && rows2 >= 0 && d >= 0, "invalid sizes");
+    if (rows1 == 0) return tpw_row_norms(x2, dtype, rows2, d, squared, norms2, stream);
+    if (rows2 == 0) return tpw_row_norms(x1, dtype, rows1, d, squared, norms1, stream);
+    TPW_REQUIRE(x1 && x2 && norms1 && norms2, "null pointer");
+    return dtype == TPW_F32 ? run(static_cast<float *>(nullptr)) : run(static_cast<uint16_t *>(nullptr));
 }
 
 extern "C" int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,

@@ -34,6 +34,8 @@
 //         grad_x2) k-major through transposing LDS reads (grad_product_bf16); other shapes
 //         write W^T and transposed x1, x2 so that both products are A . B^T with k-contiguous
 //         rows (inner_grad_gemm).
+#include <type_traits>
+
 #include "common.hpp"
 #include "tile_mfma.hpp"
 
@@ -790,10 +792,61 @@ BwdWs carve(void *ws, int64_t batch, int64_t n, int64_t m, int64_t d, size_t *to
     return w;
 }
 
+// The one-launch backward (op_backward_kernel below): tile, chunk and split plan.
+constexpr int kOpRows = 64, kOpK = 32;
+constexpr int kOpWStride = kOpRows + 2;  // floats: the transposing stores of 8 x 8 lanes on 64 banks
+
+// One direction of the launch: R rows of the gradient, K rows of the other operand.
+struct OpDir {
+    int64_t R, K, tiles_r, splits, kps, blocks;
+};
+struct OpPlan {
+    OpDir dir[2];  // grad_x1, grad_x2
+    int64_t tiles_f;
+    bool finish;
+    size_t part[2], coef[2], total;  // float offsets of the split partials and their row terms
+};
+
+OpPlan op_plan(int64_t batch, int64_t n, int64_t m, int64_t d) {
+    OpPlan P{};
+    const int64_t ft = d <= 64 ? 64 : 128;
+    P.tiles_f = cdiv(d, ft);
+    const int64_t rows[2] = {n, m};
+    const int64_t base = (cdiv(n, kOpRows) + cdiv(m, kOpRows)) * P.tiles_f * batch;
+    const int64_t fill = 2 * device_cus();
+    for (int t = 0; t < 2; ++t) {
+        OpDir &D = P.dir[t];
+        D.R = rows[t];
+        D.K = rows[1 - t];
+        D.tiles_r = cdiv(D.R, kOpRows);
+        int64_t sp = base >= fill ? 1 : fill / (base < 1 ? 1 : base);
+        // the longer K takes more of the splits: its blocks are the longer ones
+        const int64_t longer = n > m ? n : m;
+        sp = cdiv(sp * D.K, longer < 1 ? 1 : longer);
+        sp = sp > 32 ? 32 : sp < 1 ? 1 : sp;
+        D.kps = cdiv(cdiv(D.K, sp), kOpK) * kOpK;
+        D.splits = D.K > 0 ? cdiv(D.K, D.kps) : 1;
+        D.blocks = D.tiles_r * P.tiles_f * batch * D.splits;
+    }
+    // both directions finish alike, so that one pass writes both gradients
+    P.finish = P.dir[0].splits > 1 || P.dir[1].splits > 1;
+    size_t at = 0;
+    for (int t = 0; t < 2; ++t) {
+        P.part[t] = at;
+        at += P.finish ? (size_t)(P.dir[t].splits * batch * P.dir[t].R * d) : 0;
+        P.coef[t] = at;
+        at += P.finish ? (size_t)(P.dir[t].splits * batch * P.dir[t].R) : 0;
+    }
+    P.total = at;
+    return P;
+}
+
 size_t workspace_bytes(int64_t batch, int64_t n, int64_t m, int64_t d) {
     size_t total = 0;
     carve(nullptr, batch, n, m, d, &total);
-    return total;
+    // the one-launch kernel's split partials lie over the passes' arrays
+    const size_t op = align256(sizeof(float) * op_plan(batch, n, m, d).total);
+    return total > op ? total : op;
 }
 
 // x [batch, rows, d] -> xt [batch, d, rows], through a 64 x 64 LDS tile.
@@ -1511,6 +1564,470 @@ int products_f32(const float *W, const float *x1, const float *x2, int64_t batch
     return run_gemm<float, true>(W, x1, batch, m, d, n, sign, w.coef2, x2, gx2, w.part, s);
 }
 
+// ---------------------------------------------------------------------------------------
+// Small and middle problems, and shapes the kernels above do not fit: both gradients in one
+// launch (and a finish where K is split), with no weight matrix in memory.  The passes above
+// (weights, two reductions, two products) run few blocks there, each as long as a 128-row tile.
+// A block owns 64 rows x FT features of one gradient and one split of K (the other operand's
+// rows), in chunks of 32: each thread loads its pairs' grad (and res) for the next chunk while
+// the current one is multiplied, forms the weights (weight_terms) on their way to LDS and sums
+// the row terms; the other operand's chunk is staged beside them, and four waves multiply 32 rows
+// x FT / 2 features each (v_mfma_f32_32x32x2_f32, or bf16 weights, rounded as the reference rounds
+// them, on v_mfma_f32_32x32x16_bf16).  grad_x1 reads grad along its rows,
+// grad_x2 across them; blocks of both directions share the launch.  K is split until the blocks
+// fill two per CU; the finish adds the splits in order.
+// Whether the one-launch kernel takes a call that the fused kernels do not.  Its cost is the
+// weights, formed once per direction and feature tile from 128- and 256-byte pieces of grad, so
+// the passes (which form them once, with products at the matrix cores' rate) stay ahead on large
+// problems.  Forward and backward, passes -> one launch: fp32 euclidean 384 x 1624 x 118
+// 149 -> 65 us, 4096^2 x 128 218 -> 172, 2048^2 x 512 183 -> 168; even at 4096^2 x 256; cosine
+// 8000 x 4000 x 400 946 against 1730, 16383 x 8191 x 60 1480 against 1990.  bf16 700 x 900 x 100
+// 283 -> 67, 2118 x 6656 x 128 483 -> 150, 2900 x 2901 x 200 725 -> 268, 2048^2 x 512 129 -> 95;
+// 4096^2 x 512 204 against 290, 8 x 1048 x 11312 x 191 880 against 1910.
+bool op_fits(const OpPlan &P, int64_t batch, int64_t n, int64_t m) {
+    return (double)batch * (double)n * (double)m * (double)P.tiles_f <= 3.0 * 0x1p23;
+}
+
+// 1 / v within an ulp, for normal v in cos_norm_fast's range: the hardware reciprocal and a Newton step.
+__device__ __forceinline__ float rcp_newton(float v) {
+    const float y = __builtin_amdgcn_rcpf(v);
+    return __builtin_fmaf(__builtin_fmaf(-v, y, 1.0f), y, y);
+}
+
+typedef uint16_t tpw_u16x4u __attribute__((ext_vector_type(4), aligned(2)));
+// Four values at any element alignment.
+__device__ __forceinline__ floatx4 load4_any(const float *p) { return *reinterpret_cast<const floatx4u *>(p); }
+__device__ __forceinline__ floatx4 load4_any(const uint16_t *p) {
+    const tpw_u16x4u v = *reinterpret_cast<const tpw_u16x4u *>(p);
+    return floatx4{bf16_to_f32(v[0]), bf16_to_f32(v[1]), bf16_to_f32(v[2]), bf16_to_f32(v[3])};
+}
+// p[0 .. 3], zero from `count` on (count may be zero or less: nothing is read).
+template <typename T>
+__device__ __forceinline__ floatx4 load4_upto(const T *p, int64_t count) {
+    if (count >= 4) return load4_any(p);
+    floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        if (e < count) v[e] = to_f32(p[e]);
+    return v;
+}
+
+// Four bf16 values as they are stored, zero past `count` (xv of the bf16 kernel).
+__device__ __forceinline__ uint2 load4_bits_upto(const uint16_t *p, int64_t count) {
+    if (count >= 4) {
+        const tpw_u16x4u v = *reinterpret_cast<const tpw_u16x4u *>(p);
+        return __builtin_bit_cast(uint2, v);
+    }
+    uint32_t w[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        if (e < count) w[e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
+    return make_uint2(w[0], w[1]);
+}
+
+// fp32: weights and features k-major.  bf16: the weights of a row contiguous in k (16-byte MFMA
+// pieces), the features k-major, read by transposing LDS reads.
+template <typename T, int FT>
+struct OpShared {
+    float W[kOpK][kOpWStride];
+    float X[kOpK][FT + 4];
+    float coef[kOpRows];
+};
+template <int FT>
+struct OpShared<uint16_t, FT> {
+    static constexpr int kWS = kOpK + 8;  // bf16 per weight row: 80 bytes
+    union {
+        uint16_t W[kOpRows][kWS];
+        float red[16][kOpRows];  // the row terms, after the K loop
+    };
+    uint16_t X[kOpK][FT + 4];
+    float coef[kOpRows];
+};
+
+template <typename T, int MODE, int FT, bool TR>
+__device__ __forceinline__ void op_body(OpShared<T, FT> &sh, int64_t unit, const OpDir &D, int64_t tiles_f, const T *g,
+                                        const T *res, const T *own, const T *other, const float *n1, const float *n2,
+                                        int64_t n, int64_t m, int64_t d, const KerParams &kp, float sign, T *out,
+                                        float *part, float *coefpart) {
+    constexpr bool kRes = MODE == kEuclid || MODE == kSigmoid || kCosO<MODE>;
+    constexpr bool kCos = kCosAny<MODE>;
+    constexpr bool BF = sizeof(T) == 2;
+    constexpr int NI = FT / 64;             // 32-feature blocks per wave
+    constexpr int XQ = kOpK * FT / 4 / 256; // float4 of the other operand per thread and chunk
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * (FT / 2);
+    int64_t u = unit;
+    const int64_t tr = u % D.tiles_r;
+    u /= D.tiles_r;
+    const int64_t tf = u % tiles_f;
+    u /= tiles_f;
+    const int64_t split = u % D.splits, b = u / D.splits;
+    const int64_t row0 = tr * kOpRows, col0 = tf * FT;
+    const int64_t kbeg = split * D.kps, kend = kbeg + D.kps < D.K ? kbeg + D.kps : D.K;
+    const T *G = g + b * n * m, *Rs = kRes ? res + b * n * m : nullptr;
+    const T *Xo = other + b * D.K * d;
+    const float *nr = kCos ? (TR ? n2 + b * m : n1 + b * n) : nullptr;  // norms of the gradient's rows
+    const float *nk = kCos ? (TR ? n1 + b * n : n2 + b * m) : nullptr;  // and of the other operand's
+
+    // The thread's pairs of a chunk, q = 0, 1, e = 0 .. 3:
+    //   direct:     row (tid >> 3) + 32 q, k = 4 (tid & 7) + e
+    //   transposed: row 4 (tid & 15) + e,  k = (tid >> 4) + 16 q
+    const int pr = TR ? 4 * (tid & 15) : tid >> 3, pk = TR ? tid >> 4 : 4 * (tid & 7);
+    float rown[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // row norms: e (transposed) or q (direct)
+    if constexpr (kCos) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t r = row0 + pr + (TR ? e : 32 * (e & 1));
+            rown[e] = r < D.R ? nr[r] : 0.0f;
+        }
+    }
+    // Where the rows' norms allow cos_terms_fast, their reciprocals (rfast: all of the thread's)
+    float rrcp[4];
+    bool rfast = kCosO<MODE>;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        rrcp[e] = kCosO<MODE> ? rcp_newton(rown[e]) : 0.0f;
+        rfast = rfast && cos_norm_fast(rown[e]);
+    }
+    // rows_in / feats_in: all of the block's rows and features exist (the same in every thread).
+    // Whole chunks are loaded from wave-uniform pointers, which advance by chunks, and 32-bit byte
+    // offsets of the thread, which do not change (offsets that would not fit take the element
+    // path).
+    const bool rows_in = row0 + kOpRows <= D.R && (TR ? 32 : 64) * m + 64 < ((int64_t)1 << 29);
+    const bool feats_in = col0 + FT <= d && 33 * d < ((int64_t)1 << 29);
+    constexpr int kXLanes = FT / 4;
+    constexpr int kXStep = 256 / kXLanes;
+    const int xk = tid / kXLanes, xc = 4 * (tid % kXLanes);  // the thread's features, K rows xk + step q
+    uint32_t po[2], xo[XQ];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        po[q] = (uint32_t)((TR ? (pk + 16 * q) * m + pr : (pr + 32 * q) * m + pk) * (int64_t)sizeof(T));
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) xo[q] = (uint32_t)(((xk + kXStep * q) * d + xc) * (int64_t)sizeof(T));
+    const T *Gc = G + (TR ? kbeg * m + row0 : row0 * m + kbeg), *Rc = kRes ? Rs + (Gc - G) : nullptr;
+    const T *Xc = Xo + kbeg * d + col0;
+    const int64_t pstep = TR ? kOpK * m : kOpK, xstep = kOpK * d;
+    auto at = [](const T *base, uint32_t bytes) {
+        return reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
+    };
+    // how many of the thread's four rows (transposed) / features exist, 0 .. 4 or more
+    const int64_t rleft = D.R - row0 - pr, xleft = d - col0 - xc;
+    typedef typename std::conditional<BF, uint2, floatx4>::type XV;
+    floatx4 gv[2], av[2], kn[2];
+    XV xv[XQ];
+    auto load_x = [&](const T *p, int64_t cnt) {
+        if constexpr (BF) return load4_bits_upto(p, cnt);
+        else return load4_upto(p, cnt);
+    };
+    // the chunk at k0 (the pointers' chunk): `left` of its 32 K rows exist
+    auto load = [&](int64_t k0, int left) {
+        if (rows_in && left == kOpK) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                gv[q] = load4_any(at(Gc, po[q]));
+                av[q] = kRes ? load4_any(at(Rc, po[q])) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (kCos) {
+                    if constexpr (TR) kn[q][0] = nk[k0 + pk + 16 * q];
+                    else kn[q] = load4_any(nk + k0 + pk);
+                }
+            }
+        } else {
+            int p = pk;  // opaque: keeps these addresses out of the whole chunks' loop
+            asm volatile("" : "+v"(p));
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int64_t cnt = TR ? (p + 16 * q < left ? rleft : 0) : (rleft > 32 * q ? left - p : 0);
+                const int64_t o = cnt > 0 ? (TR ? (p + 16 * q) * m + pr : (pr + 32 * q) * m + p) : 0;
+                gv[q] = load4_upto(Gc + o, cnt);
+                av[q] = kRes ? load4_upto(Rc + o, cnt) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (kCos) {
+                    if constexpr (TR) kn[q][0] = p + 16 * q < left ? nk[k0 + p + 16 * q] : 0.0f;
+                    else kn[q] = load4_upto(nk + k0 + (p < left ? p : 0), left - p);
+                }
+            }
+        }
+        if (feats_in && left == kOpK) {
+#pragma unroll
+            for (int q = 0; q < XQ; ++q) xv[q] = load_x(at(Xc, xo[q]), 4);
+        } else {
+            int x = xk;
+            asm volatile("" : "+v"(x));
+#pragma unroll
+            for (int q = 0; q < XQ; ++q) {
+                const int64_t cnt = x + kXStep * q < left ? xleft : 0;
+                xv[q] = load_x(Xc + (cnt > 0 ? (x + kXStep * q) * d + xc : 0), cnt);
+            }
+        }
+        Gc += pstep;
+        if constexpr (kRes) Rc += pstep;
+        Xc += xstep;
+    };
+    float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // row terms: e (transposed) or q (direct)
+    auto store = [&](int left) {
+        const bool whole = rows_in && left == kOpK;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            float w[4], t[4];  // weights and row terms
+            bool fast = rfast;
+            if constexpr (kCosO<MODE>) {
+#pragma unroll
+                for (int e = 0; e < (TR ? 1 : 4); ++e) fast = fast && cos_norm_fast(kn[q][e]);
+            }
+            if (kCosO<MODE> && fast) {
+                if constexpr (kCosO<MODE>) {
+                    float kr[4];
+#pragma unroll
+                    for (int e = 0; e < (TR ? 1 : 4); ++e) kr[e] = rcp_newton(kn[q][e]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float vr = rrcp[TR ? e : q], vk = kr[TR ? 0 : e];
+                        float rt, ct;
+                        cos_terms_fast<MODE>(gv[q][e], av[q][e], TR ? vk : vr, TR ? vr : vk, w[e], rt, ct);
+                        t[e] = TR ? ct : rt;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float vr = rown[TR ? e : q], vk = kCos ? kn[q][TR ? 0 : e] : 0.0f;
+                    float rt, ct;
+                    weight_terms<MODE, BF>(gv[q][e], av[q][e], TR ? vk : vr, TR ? vr : vk, kp, w[e], rt, ct);
+                    t[e] = TR ? ct : rt;
+                }
+            }
+            if (!whole) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool in = TR ? e < rleft && pk + 16 * q < left : 32 * q < rleft && pk + e < left;
+                    w[e] = in ? w[e] : 0.0f;
+                    t[e] = in ? t[e] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rs[TR ? e : q] += t[e];
+            if constexpr (BF) {
+                const uint2 hw = make_uint2(f32x2_to_bf16x2_rne(w[0], w[1]), f32x2_to_bf16x2_rne(w[2], w[3]));
+                if constexpr (TR) {
+                    sh.W[pr][pk + 16 * q] = (uint16_t)hw.x;
+                    sh.W[pr + 1][pk + 16 * q] = (uint16_t)(hw.x >> 16);
+                    sh.W[pr + 2][pk + 16 * q] = (uint16_t)hw.y;
+                    sh.W[pr + 3][pk + 16 * q] = (uint16_t)(hw.y >> 16);
+                } else {
+                    *reinterpret_cast<uint2 *>(&sh.W[pr + 32 * q][pk]) = hw;
+                }
+            } else if constexpr (TR) {
+                float *dst = &sh.W[pk + 16 * q][pr];
+                *reinterpret_cast<float2 *>(dst) = make_float2(w[0], w[1]);
+                *reinterpret_cast<float2 *>(dst + 2) = make_float2(w[2], w[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sh.W[pk + e][pr + 32 * q] = w[e];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < XQ; ++q) *reinterpret_cast<XV *>(&sh.X[xk + kXStep * q][xc]) = xv[q];
+    };
+
+    floatx16 acc[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[ni][r] = 0.0f;
+    // Sums over more than kOpFlush of K are blocked: the running accumulators are added to a second
+    // set and restart, which keeps the rounding of long sums where the split passes had it.
+    constexpr int kOpFlush = 512;
+    floatx16 tot[NI];
+    float rtot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) tot[ni] = acc[ni];
+    auto flush = [&]() {
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                tot[ni][r] += acc[ni][r];
+                acc[ni][r] = 0.0f;
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            rtot[e] += rs[e];
+            rs[e] = 0.0f;
+        }
+    };
+    auto left_of = [&](int64_t k0) { return kend - k0 < kOpK ? (int)(kend - k0) : kOpK; };
+    if (kbeg < kend) load(kbeg, left_of(kbeg));
+    for (int64_t k0 = kbeg; k0 < kend; k0 += kOpK) {
+        if (k0 > kbeg && (k0 - kbeg) % kOpFlush == 0) flush();
+        store(left_of(k0));
+        __syncthreads();
+        if (k0 + kOpK < kend) load(k0 + kOpK, left_of(k0 + kOpK));
+        if constexpr (BF) {
+#pragma unroll
+            for (int st = 0; st < kOpK / 16; ++st) {
+                // k = 16 st + 8 h .. + 7 of the lane's row, and of its feature: two transposing reads
+                // of four K rows each (lane j of a group of 16 points at four features of one K
+                // row; lane i receives the four K rows of feature i)
+                const uint4 a = *reinterpret_cast<const uint4 *>(&sh.W[wr + l32][16 * st + 8 * h]);
+                const int j = lane & 15, f0 = 16 * ((lane >> 4) & 1) + 4 * (j & 3);
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) {
+                    typedef short v4s __attribute__((ext_vector_type(4)));
+                    uint2 v[2];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const uint16_t *p = &sh.X[16 * st + 8 * h + 4 * t + (j >> 2)][wc + 32 * ni + f0];
+                        const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (__attribute__((address_space(3))) v4s *)(uintptr_t)tile::lds_addr(p));
+                        v[t] = __builtin_bit_cast(uint2, r);
+                    }
+                    acc[ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, a),
+                        __builtin_bit_cast(bf16x8, make_uint4(v[0].x, v[0].y, v[1].x, v[1].y)), acc[ni], 0, 0, 0);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int st = 0; st < kOpK / 2; ++st) {
+                const int kk = 2 * st + h;
+                const float a = sh.W[kk][wr + l32];
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni)
+                    acc[ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, sh.X[kk][wc + 32 * ni + l32], acc[ni], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    flush();
+
+    // the rows' terms over the threads that share a row, in a fixed order: eight neighbouring lanes
+    // (direct), or threads 16 apart through LDS (transposed)
+    if constexpr (TR) {
+        float *red;  // 16 x 64, free after the loop's last barrier
+        if constexpr (BF) red = &sh.red[0][0];
+        else red = &sh.W[0][0];
+        static_assert(16 * kOpRows <= kOpK * kOpWStride, "the row terms fit in W");
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[(tid >> 4) * kOpRows + pr + e] = rtot[e];
+        __syncthreads();
+        if (tid < kOpRows) {
+            float t = red[tid];
+#pragma unroll
+            for (int q = 1; q < 16; ++q) t += red[q * kOpRows + tid];
+            sh.coef[tid] = t;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            float t = rtot[q];
+            t += __shfl_xor(t, 4, 64);
+            t += __shfl_xor(t, 2, 64);
+            t += __shfl_xor(t, 1, 64);
+            if ((tid & 7) == 0) sh.coef[pr + 32 * q] = t;
+        }
+    }
+    __syncthreads();
+    const int64_t prow = (part ? (b * D.splits + split) : b) * D.R;  // first row of this block's array
+    if (part && tf == 0 && tid < kOpRows && row0 + tid < D.R) coefpart[prow + row0 + tid] = sh.coef[tid];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+        const int64_t col = col0 + wc + 32 * ni + l32;
+        if (col >= d) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int rr = wr + 8 * (r >> 2) + 4 * h + (r & 3);
+            const int64_t row = row0 + rr;
+            if (row >= D.R) continue;
+            const int64_t o = (prow + row) * d + col;
+            if (part) {
+                part[o] = tot[ni][r];
+            } else {
+                float c = sh.coef[rr];
+                if constexpr (kCos) {
+                    const float nv = nr[row];
+                    c = nv == 0.0f ? 0.0f : __fdiv_rn(c, nv);
+                }
+                from_f32(out + o, __builtin_fmaf(c, to_f32(own[o]), sign * tot[ni][r]));
+            }
+        }
+    }
+}
+
+template <typename T, int MODE, int FT>
+__global__ __launch_bounds__(256, 2) void op_backward_kernel(
+    const T *__restrict__ g, const T *__restrict__ res, const T *__restrict__ x1, const T *__restrict__ x2,
+    const float *__restrict__ n1, const float *__restrict__ n2, int64_t n, int64_t m, int64_t d, OpDir d1, OpDir d2,
+    int64_t tiles_f, KerParams kp, float sign, T *__restrict__ gx1, T *__restrict__ gx2, float *part1, float *coef1,
+    float *part2, float *coef2) {
+    __shared__ OpShared<T, FT> sh;
+    const int64_t bid = blockIdx.x;
+    if (bid < d1.blocks)
+        op_body<T, MODE, FT, false>(sh, bid, d1, tiles_f, g, res, x1, x2, n1, n2, n, m, d, kp, sign, gx1, part1, coef1);
+    else
+        op_body<T, MODE, FT, true>(sh, bid - d1.blocks, d2, tiles_f, g, res, x2, x1, n1, n2, n, m, d, kp, sign, gx2,
+                                   part2, coef2);
+}
+
+// Both gradients from the splits' partials [batch, splits, R, d] and row terms [batch, splits, R].
+template <typename T>
+__global__ __launch_bounds__(256) void op_finish_kernel(const float *__restrict__ part1,
+                                                        const float *__restrict__ coef1,
+                                                        const float *__restrict__ part2,
+                                                        const float *__restrict__ coef2, const T *__restrict__ x1,
+                                                        const T *__restrict__ x2, const float *__restrict__ n1,
+                                                        const float *__restrict__ n2, int64_t batch, int64_t d,
+                                                        int64_t n, int64_t s1, int64_t m, int64_t s2, float sign,
+                                                        T *__restrict__ gx1, T *__restrict__ gx2) {
+    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t len1 = batch * n * d;
+    const bool two = t >= len1;
+    if (two) t -= len1;
+    const int64_t R = two ? m : n, splits = two ? s2 : s1;
+    if (t >= batch * R * d) return;
+    const float *part = two ? part2 : part1, *cp = two ? coef2 : coef1, *nv = two ? n2 : n1;
+    const int64_t row = t / d, b = row / R, r = row - b * R, k = t - row * d;  // row: of all batches
+    const float *p = part + (b * splits * R + r) * d + k;
+    const float *c = cp + b * splits * R + r;
+    float s = p[0], co = c[0];
+    int64_t q = 1;
+    for (; q + 4 <= splits; q += 4) {
+        float v[4], w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p[(q + e) * R * d], w[e] = c[(q + e) * R];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += v[e], co += w[e];
+    }
+    for (; q < splits; ++q) s += p[q * R * d], co += c[q * R];
+    if (nv) {
+        const float v = nv[row];
+        co = v == 0.0f ? 0.0f : __fdiv_rn(co, v);
+    }
+    const T *own = two ? x2 : x1;
+    T *out = two ? gx2 : gx1;
+    from_f32(out + t, __builtin_fmaf(co, to_f32(own[t]), sign * s));
+}
+
+template <typename T, int MODE>
+int run_op_backward(const OpPlan &P, const T *g, const T *x1, const T *x2, const T *res, const float *n1,
+                    const float *n2, int64_t batch, int64_t n, int64_t m, int64_t d, T *gx1, T *gx2, float *ws,
+                    hipStream_t s, KerParams kp) {
+    const float sign = (MODE == kEuclid || MODE == kSqEuclid) ? -1.0f : 1.0f;
+    float *p1 = P.finish ? ws + P.part[0] : nullptr, *c1 = P.finish ? ws + P.coef[0] : nullptr;
+    float *p2 = P.finish ? ws + P.part[1] : nullptr, *c2 = P.finish ? ws + P.coef[1] : nullptr;
+    const dim3 grid((unsigned)(P.dir[0].blocks + P.dir[1].blocks));
+    if (d <= 64)
+        hipLaunchKernelGGL((op_backward_kernel<T, MODE, 64>), grid, dim3(256), 0, s, g, res, x1, x2, n1, n2, n, m, d,
+                           P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
+    else
+        hipLaunchKernelGGL((op_backward_kernel<T, MODE, 128>), grid, dim3(256), 0, s, g, res, x1, x2, n1, n2, n, m, d,
+                           P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
+    const int rc = check_launch("op_backward_kernel");
+    if (rc != TPW_OK || !P.finish) return rc;
+    hipLaunchKernelGGL(op_finish_kernel<T>, dim3((unsigned)cdiv(batch * (n + m) * d, 256)), dim3(256), 0, s, p1, c1,
+                       p2, c2, x1, x2, kCosAny<MODE> ? n1 : nullptr, kCosAny<MODE> ? n2 : nullptr, batch, d, n,
+                       P.dir[0].splits, m, P.dir[1].splits, sign, gx1, gx2);
+    return check_launch("op_finish_kernel");
+}
+
 template <typename T, int MODE>
 int run_backward(const T *g, const T *x1, const T *x2, const T *res, const float *n1,
                  const float *n2, int dtype, int64_t batch, int64_t n, int64_t m, int64_t d, T *gx1,
@@ -1539,6 +2056,10 @@ int run_backward(const T *g, const T *x1, const T *x2, const T *res, const float
         }
     }
     if constexpr (MODE == kDot && !kBf16) {
+        const OpPlan P = op_plan(batch, n, m, d);
+        if (op_fits(P, batch, n, m) && !tile_grid_fills(batch, n, d))
+            return run_op_backward<T, MODE>(P, g, x1, x2, res, n1, n2, batch, n, m, d, gx1, gx2,
+                                            static_cast<float *>(ws), s, kp);
         // fp32: grad is the weight matrix as stored; no weight pass, zero coefficients
         hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)cdiv(2 * batch * n, 256)), dim3(256), 0, s,
                            reinterpret_cast<uint16_t *>(w.coef1), 2 * batch * n);
@@ -1666,6 +2187,12 @@ int run_backward(const T *g, const T *x1, const T *x2, const T *res, const float
                                n2, batch * m, d);
             return check_launch("cos_proj_finish_kernel");
         }
+    }
+    if constexpr (!kCosMode && MODE != kPoly) {
+        const OpPlan P = op_plan(batch, n, m, d);
+        if (op_fits(P, batch, n, m))
+            return run_op_backward<T, MODE>(P, g, x1, x2, res, n1, n2, batch, n, m, d, gx1, gx2,
+                                            static_cast<float *>(ws), s, kp);
     }
     int64_t ti = cdiv(n, kPWRows);
     int64_t tj = cdiv(m, kPWCols);

@@ -98,12 +98,14 @@ at::Tensor pw_inner_cuda(const at::Tensor &x1, const at::Tensor &x2, int64_t epi
     if (epilogue != TPW_EPI_DOT && !small) {
         const int squared = (epilogue == TPW_EPI_EUCLIDEAN || epilogue == TPW_EPI_SQEUCLIDEAN);
         n1 = at::empty({B, n}, a.options().dtype(at::kFloat));
-        check_rc(tpw_row_norms(a.data_ptr(), dt, B * n, d, squared, n1.data_ptr<float>(), s), "row norms");
         if (x2.is_same(x1)) {
+            check_rc(tpw_row_norms(a.data_ptr(), dt, B * n, d, squared, n1.data_ptr<float>(), s), "row norms");
             n2 = n1;  // x2 = None: one set of norms
         } else {
             n2 = at::empty({B, m}, a.options().dtype(at::kFloat));
-            check_rc(tpw_row_norms(b.data_ptr(), dt, B * m, d, squared, n2.data_ptr<float>(), s), "row norms");
+            check_rc(tpw_row_norms2(a.data_ptr(), B * n, b.data_ptr(), B * m, dt, d, squared, n1.data_ptr<float>(),
+                                    n2.data_ptr<float>(), s),
+                     "row norms");
         }
     }
     // Rows that are not whole 128-byte chunks (or operands not 16-byte aligned) would take the
@@ -165,8 +167,9 @@ std::tuple<at::Tensor, at::Tensor> pw_inner_backward_cuda(const at::Tensor &grad
                epilogue == TPW_EPI_CORRELATION) {
         auto n1 = at::empty({B, n}, a.options().dtype(at::kFloat));
         auto n2 = at::empty({B, m}, a.options().dtype(at::kFloat));
-        check_rc(tpw_row_norms(a.data_ptr(), dt, B * n, d, 0, n1.data_ptr<float>(), s), "row norms");
-        check_rc(tpw_row_norms(b.data_ptr(), dt, B * m, d, 0, n2.data_ptr<float>(), s), "row norms");
+        check_rc(tpw_row_norms2(a.data_ptr(), B * n, b.data_ptr(), B * m, dt, d, 0, n1.data_ptr<float>(),
+                                n2.data_ptr<float>(), s),
+                 "row norms");
         // the forward's output, when autograd saved it: the weights come from it
         at::Tensor o = res.defined() ? res.reshape({B, n, m}).contiguous() : at::Tensor();
         check_rc(tpw_cosine_backward(g.data_ptr(), a.data_ptr(), b.data_ptr(), n1.data_ptr<float>(),
