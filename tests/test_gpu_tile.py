@@ -86,6 +86,8 @@ def test_inner_tile_kernel_equals_staged_kernel(dtype, B, n, m, d, epi):
 # bf16 rounding), and a tile with a zero row divides: one bf16 ulp between the two.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,m,d", [(64, 64, 64), (65, 63, 50), (1, 129, 1), (33, 100, 128), (130, 7, 257),
+                                   # the tile kernel with ragged rows (16-byte units at any alignment)
+                                   (65, 63, 64), (130, 131, 128), (40, 1, 64), (129, 142, 1024),
                                    (40, 66, 100), (31, 32, 516)])
 @pytest.mark.parametrize("epi", EPIS)
 def test_small_output_kernel_equals_tile_kernels(dtype, n, m, d, epi):

@@ -517,7 +517,7 @@ __global__ __launch_bounds__(kThreads, 2) void pairwise_inner_kernel(
 // row-segment stores.  AK / BK: x1 / x2 stored k-major, [d, n] / [d, m] (the backward's products
 // read W^T, x1 and x2 that way, without a transposed copy); bf16 k-major pieces come from two
 // transposing LDS reads each.
-// RG: bf16 output rows of m % 8 != 0 values (store_tile's ragged mode), a separate
+// RG: output rows that are no whole 16-byte units (store_tile's ragged mode), a separate
 // instantiation so that the aligned kernels' code is unchanged by it.
 template <typename T, typename OutT, int EPI, int NB = 1, bool AK = false, bool BK = false, bool RG = false>
 __global__ __launch_bounds__(tile::kThreads, NB == 1 ? 4 : 2) void inner_tile_kernel(
@@ -709,7 +709,7 @@ __global__ __launch_bounds__(tile::kThreads, NB == 1 ? 4 : 2) void inner_tile_ke
             }
             return o;
         },
-        out, b, row0, col0, n, m, RG);
+        out, b, row0, col0, n, m, RG ? kRaggedUnits : 0);
     }
 }
 
@@ -1091,11 +1091,10 @@ int launch_inner(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, 
     const bool direct = vec && d % Elem<T>::kChunk == 0 && d > 0 && (n > m ? n : m) * d < ((int64_t)1 << 31);
     if constexpr (EPI != kEpiPoly) {
         // the tile kernel: byte offsets below 2^32, whole 16-byte units per output row (and, for
-        // the gradient products, 16-byte aligned X rows).  bf16 outputs of the distance
-        // epilogues also take ragged rows (store_tile's unit + head / tail stores).  Ragged fp32
-        // rows stay on the staged kernel: the tile store's dword rows cost the matrix-core-bound
-        // products more (16384 x 16383 x 128 euclidean 0.676 -> 0.716 ms)
-        constexpr bool kRaggedOk = sizeof(OutT) == 2 && EPI != kEpiGrad && EPI != kEpiGradA;
+        // the gradient products, 16-byte aligned X rows).  The distance epilogues
+        // also take ragged rows (store_tile's unaligned units): fp32 16384 x 16383 x 128 674 -> 645 us
+        // a call against the staged kernel, 10007 x 10006 x 50 197 -> 172.
+        constexpr bool kRaggedOk = sizeof(OutT) >= 2 && sizeof(OutT) <= 4 && EPI != kEpiGrad && EPI != kEpiGradA;
         if (direct && (n > m ? n : m) * d * (int64_t)sizeof(T) < ((int64_t)1 << 32) && aligned16(out) &&
             (m % (16 / (int64_t)sizeof(OutT)) == 0 || kRaggedOk) && (EPI != kEpiGrad || aligned16(X))) {
             const LaunchEvents ev = launch_events("inner_tile_kernel");

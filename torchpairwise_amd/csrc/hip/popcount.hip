@@ -818,15 +818,16 @@ __device__ __forceinline__ void pops_to_float(bool small, uint32_t *s_pop) {
 // products: register 4 g + e of lane l32 + 32 h in block (mi, ni) is row wr + 32 mi + l32,
 // column wc + 32 ni + 8 g + 4 h + e of the tile).  Rows of at most kSmallRowLimit features
 // finish in float (finish_small, popcounts already floats in s_pop), longer rows on integer
-// counts (finish); both give the same bits.  Any m: rows of m % 4 != 0 floats are written a
-// dword per lane (the ragged mode of tile::store_tile), a separate instantiation (RAGGED) so
-// that the aligned kernels' code is unchanged by it.
+// counts (finish); both give the same bits.  Any m: rows of m % 4 != 0 floats take a ragged mode
+// of tile::store_tile, a separate instantiation (RAGGED) so that the aligned kernels' code is
+// unchanged by it.
 template <int OP, int EPI, bool RAGGED>
 __device__ __forceinline__ void bool_tile_store(bool small, const floatx16 (&facc)[2][2], uint4 *smem,
                                                 const uint32_t *s_pop, int wr, int wc, int l32, int h, int64_t d,
                                                 double inv_d, float inv_df, float *__restrict__ out, int64_t b,
                                                 int64_t row0, int64_t col0, int64_t n, int64_t m) {
     using tile::kT;
+    constexpr int kRaggedMode = !RAGGED ? 0 : EPI < kJaccard ? tile::kRaggedRows : tile::kRaggedUnits;
     const float df = (float)d;
     if (small) {
         float pav[2];
@@ -843,7 +844,7 @@ __device__ __forceinline__ void bool_tile_store(bool small, const floatx16 (&fac
                 for (int e = 0; e < 4; ++e) o[e] = finish_small<OP, EPI>(facc[mi][ni][4 * g + e], pav[mi], pbe[e], df, inv_df);
                 return o;
             },
-            out, b, row0, col0, n, m, RAGGED);
+            out, b, row0, col0, n, m, kRaggedMode);
         return;
     }
     const uint32_t du = (uint32_t)d;
@@ -863,7 +864,7 @@ __device__ __forceinline__ void bool_tile_store(bool small, const floatx16 (&fac
             }
             return o;
         },
-        out, b, row0, col0, n, m, RAGGED);
+        out, b, row0, col0, n, m, kRaggedMode);
 }
 
 template <int OP, int EPI, bool RAGGED>

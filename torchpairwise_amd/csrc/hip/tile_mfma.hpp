@@ -224,13 +224,16 @@ __device__ __forceinline__ void store16(V *p, V v) {
 // workgroup barrier), written as (NI * 128)-byte row segments, 8 NI lanes per row.  value(ni,
 // g) returns the lane's register quad g of block ni: row grow0 + l32, columns gcol0 + 32 ni +
 // 8 g + 4 h + (0..3).  Rows >= n and columns >= m are not stored (m a multiple of 4, out
-// 16-byte aligned).  Stage unit u of row r sits at u ^ (r & 15).  With `ragged` (rows of
-// m % 4 != 0 floats, so no 16-byte row segments) each store instruction writes one row's
-// 32 NI values instead, a dword per lane: 128 NI contiguous bytes, 32 instructions per slice.
+// 16-byte aligned).  Stage unit u of row r sits at u ^ (r & 15).  `ragged` takes any m:
+// kRaggedUnits the same units at dword-aligned addresses, as plain stores; kRaggedRows one row's
+// 32 NI values per store instruction, a dword per lane (128 NI contiguous bytes, 32 instructions
+// per slice), faster for kernels that do little but store (hamming 16384 x 16383 x 500: 303
+// against 314 us) and slower for the others (jaccard at d = 1024: 318 -> 289 us by units).
+constexpr int kRaggedUnits = 1, kRaggedRows = 2;
 template <int NI, bool kNT = true, class F>
 __device__ __forceinline__ void store_wave_rows_f32(floatx4 *sl, F &&value, float *__restrict__ out, int64_t b,
                                                     int64_t grow0, int64_t gcol0, int64_t n, int64_t m,
-                                                    bool ragged = false) {
+                                                    int ragged = 0) {
     constexpr int U = NI * 8;    // 16-byte units per stage row
     constexpr int RPI = 64 / U;  // rows per store instruction
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
@@ -244,7 +247,7 @@ __device__ __forceinline__ void store_wave_rows_f32(floatx4 *sl, F &&value, floa
         }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
-    if (ragged) {
+    if (ragged == kRaggedRows) {
         const float *sf = reinterpret_cast<const float *>(sl);
         const int c = lane % (32 * NI);
         const int64_t gcol = gcol0 + c;
@@ -254,6 +257,24 @@ __device__ __forceinline__ void store_wave_rows_f32(floatx4 *sl, F &&value, floa
             const float v = sf[(r * U + ((c >> 2) ^ (r & 15))) * 4 + (c & 3)];
             const int64_t grow = grow0 + r;
             if (col_ok && grow < n) store16<kNT>(out + (b * n + grow) * m + gcol, v);
+        }
+    } else if (ragged == kRaggedUnits) {
+        // 16 bytes at a dword-aligned address, which global memory takes; plain stores, so that the
+        // L2 joins the neighbouring pieces of a line before it leaves
+        const int64_t gcol = gcol0 + 4 * ul;
+#pragma unroll
+        for (int it = 0; it < 32 / RPI; ++it) {
+            const int r = it * RPI + rl;
+            const floatx4 v = sl[r * U + (ul ^ (r & 15))];
+            const int64_t grow = grow0 + r;
+            float *p = out + (b * n + grow) * m + gcol;
+            if (grow < n && gcol + 3 < m) {
+                *reinterpret_cast<floatx4u *>(p) = v;
+            } else if (grow < n) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (gcol + e < m) p[e] = v[e];
+            }
         }
     } else {
         const int64_t gcol = gcol0 + 4 * ul;
@@ -307,14 +328,15 @@ __device__ __forceinline__ void store_wave_rows_bf16(uint4 *sl, F &&value, uint1
 // wr + 32 mi + l32, columns wc + 32 ni + 8 g + 4 h + (0..3).  Rows >= n and columns >= m are not
 // stored; m must be a multiple of 16 / sizeof(OutT) and out 16-byte aligned (a 16-byte store
 // unit is then wholly inside or outside), except that fp32 and bf16 outputs take any m with
-// `ragged` set (fp32: dword row stores, store_wave_rows_f32; bf16: whole 16-byte units
-// funnel-shifted from the stage, 2-byte stores for each row piece's head and tail).  bf16 stages the rounded values of the whole tile (one
+// `ragged` set (kRaggedUnits or, fp32 only, kRaggedRows: see store_wave_rows_f32; bf16
+// units funnel-shifted to aligned addresses, with 2-byte stores for each row piece's head and
+// tail, took 825 us where unaligned units take 471: euclidean 8 x 8192 x 8191 x 256).  bf16 stages the rounded values of the whole tile (one
 // pass of 128 rows x 256 bytes, one workgroup barrier); fp32 per wave (store_wave_rows_f32, an
 // 8 KiB slice each).  Stage unit u of row r sits at u ^ (r & 15): conflict-free 16-byte accesses
 // across 16 rows and within 16-unit groups.
 template <typename OutT, bool kNT = true, class F>
 __device__ __forceinline__ void store_tile(uint4 *st, F &&value, OutT *__restrict__ out, int64_t b, int64_t row0,
-                                           int64_t col0, int64_t n, int64_t m, bool ragged = false) {
+                                           int64_t col0, int64_t n, int64_t m, int ragged = 0) {
     if constexpr (sizeof(OutT) == 4) {
         const int wave = threadIdx.x >> 6;
         const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
@@ -371,43 +393,23 @@ __device__ __forceinline__ void store_tile(uint4 *st, F &&value, OutT *__restric
         barrier_lds();
         if constexpr (sizeof(OutT) == 2) {
             if (ragged) {
-                // rows of m % 8 != 0 values: a row piece starts anywhere inside a 16-byte unit
-                // (out itself 16-byte aligned).  16 lanes per row write the piece's whole units,
-                // each funnel-shifted from two stage units; then 16 lanes per row its head and
-                // tail values (at most 7 + 7), 2 bytes each.
-                static_assert(NPASS == 1 && RPI == 4, "bf16 stage geometry");
-                const int j = lane & 15, rq = lane >> 4;
-                const uint16_t *sh = reinterpret_cast<const uint16_t *>(st);
-                const int V = (int)(m - col0 < kT ? m - col0 : kT);  // values in the piece
-#pragma unroll 2
-                for (int it = 0; it < ITERS; ++it) {
-                    const int r = (wave * ITERS + it) * RPI + rq;
-                    const int64_t grow = row0 + r;
-                    if (grow >= n) continue;
-                    const int64_t e0 = (b * n + grow) * m + col0;  // the piece's first value
-                    const int sft = (int)((8 - (e0 & 7)) & 7);     // values before the first unit
-                    const int K = V > sft ? (V - sft) >> 3 : 0;    // whole units
-                    if (j < K) {
-                        const int c0 = sft + 8 * j, u0 = c0 >> 3;  // value c0 sits at c0 & 7 = sft
-                        const u32x4 A = reinterpret_cast<const u32x4 *>(st)[r * UPR + (u0 ^ (r & XM))];
-                        const u32x4 B = sft != 0 ? reinterpret_cast<const u32x4 *>(st)[r * UPR + ((u0 + 1) ^ (r & XM))] : A;
-                        const uint32_t w[8] = {A[0], A[1], A[2], A[3], B[0], B[1], B[2], B[3]};
-                        const int q = sft >> 1;
-                        u32x4 o;
+                // rows of m % 8 != 0 values: 16 bytes at a 2-byte aligned address, which global
+                // memory takes, as plain stores (see store_wave_rows_f32)
+                typedef uint32_t u32x4h __attribute__((ext_vector_type(4), aligned(2)));
+                const int ul = lane % LPR, rl = lane / LPR;
+                const int64_t gcol = col0 + 8 * ul;
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            const uint32_t lo = q == 0 ? w[k] : q == 1 ? w[k + 1] : q == 2 ? w[k + 2] : w[k + 3];
-                            const uint32_t hi = q == 0 ? w[k + 1] : q == 1 ? w[k + 2] : q == 2 ? w[k + 3] : w[k + 4];
-                            o[k] = (sft & 1) ? (lo >> 16) | (hi << 16) : lo;
-                        }
-                        store16<kNT>(reinterpret_cast<u32x4 *>(out + e0 + c0), o);
-                    }
-                    const int headN = sft < V ? sft : V, tail0 = sft + 8 * K;
-                    const int tailN = V > tail0 ? V - tail0 : 0;
-                    if (j < headN + tailN) {
-                        const int c = j < headN ? j : tail0 + (j - headN);
-                        store16<kNT>(reinterpret_cast<uint16_t *>(out + e0 + c),
-                                     sh[(r * UPR + ((c >> 3) ^ (r & XM))) * 8 + (c & 7)]);
+                for (int it = 0; it < ITERS; ++it) {
+                    const int r = (wave * ITERS + it) * RPI + rl;
+                    const u32x4 v = reinterpret_cast<const u32x4 *>(st)[r * UPR + (ul ^ (r & XM))];
+                    const int64_t grow = row0 + pass * PR + r;
+                    OutT *p = out + (b * n + grow) * m + gcol;
+                    if (grow < n && gcol + 7 < m) {
+                        *reinterpret_cast<u32x4h *>(p) = v;
+                    } else if (grow < n) {
+#pragma unroll
+                        for (int e = 0; e < 7; ++e)
+                            if (gcol + e < m) p[e] = (OutT)(v[e >> 1] >> (16 * (e & 1)));
                     }
                 }
                 return;
