@@ -69,10 +69,10 @@ def test_jaccard_bit_exact(B, n, m, d):
     assert_equal(got, torch.from_numpy(want_c), "jaccard vs C passes")
 
 
-# rows of at most 8 words and m % 4 != 0: the 32 x 512 tile with dword row stores, at the edges of
-# its column groups (64), tile width (512) and rows (32), with and without row popcounts
-@pytest.mark.parametrize("m", [257, 319, 321, 511, 513, 1089])
-@pytest.mark.parametrize("B,n,d", [(1, 1, 1), (2, 33, 166), (1, 64, 256)])
+# rows of at most 8 words and m % 4 != 0: the 32 x 512 tile of rows 32 apart, at the edges of its
+# tile width (512), of the widest with its 31 columns of lead (481) and of its rows (256)
+@pytest.mark.parametrize("m", [257, 319, 321, 481, 511, 513, 993, 1089])
+@pytest.mark.parametrize("B,n,d", [(1, 1, 1), (2, 33, 166), (1, 64, 256), (2, 257, 100), (1, 555, 128)])
 def test_bool_ragged_rows_bit_exact(B, n, m, d):
     x1, x2 = rand(B, n, d, seed=7) < 0.4, rand(B, m, d, seed=8) < 0.4
     x2[:, :3] = False
@@ -80,6 +80,20 @@ def test_bool_ragged_rows_bit_exact(B, n, m, d):
     assert_equal(got, torch.from_numpy(P.pw_reduce_bool(x1.numpy(), x2.numpy(), "eq", "mean")), f"eq mean m={m}")
     assert_equal(capi.jaccard_bool(x1.to(DEV), x2.to(DEV)),
                  torch.from_numpy(P.jaccard_distances(x1.numpy(), x2.numpy())), f"jaccard m={m}")
+
+
+@pytest.mark.parametrize("offset,m", [(1, 512), (2, 516), (3, 1000), (1, 515)])
+def test_bool_ragged_rows_unaligned_output(offset, m):
+    """Outputs that begin inside a line: nothing outside the rows is written."""
+    B, n, d = 2, 70, 166
+    x1, x2 = rand(B, n, d, seed=7) < 0.4, rand(B, m, d, seed=8) < 0.4
+    w1, w2 = capi.pack_bool(x1.to(DEV))[0], capi.pack_bool(x2.to(DEV))[0]
+    buf = torch.full((offset + B * n * m + 5,), -7.0, device=DEV)
+    out = buf[offset:offset + B * n * m]
+    capi.call("tpw_bool_pairwise_reduce", capi._ptr(w1), capi._ptr(w2), B, n, m, d, capi.BIT_NE, capi.RED_SUM,
+              capi._ptr(out), capi._stream())
+    assert_equal(out.view(B, n, m), torch.from_numpy(P.pw_reduce_bool(x1.numpy(), x2.numpy(), "ne", "sum")), "ne sum")
+    assert bool((buf[:offset] == -7).all()) and bool((buf[offset + B * n * m:] == -7).all())
 
 
 def test_bool_empty_sizes():

@@ -256,11 +256,14 @@ __device__ __forceinline__ uint32_t popacc(uint32_t acc, uint4 a, uint4 b) {
 // CV uint4 (4 words) per row and LDS chunk.  128 x 128 (TX = 16) for general rows; 32 x 512
 // (TX = 64) for rows of at most 8 words, where the output write is the whole cost and 2 KB
 // contiguous per row and tile keep the DRAM pages open longer than 512 B.
-// RAGGED (TX = 64, rows of m % 4 != 0 floats or an unaligned output, which no 16-byte store
-// fits): thread tx owns columns tx + 64 j instead, so each dword store instruction of a wave
-// covers 256 contiguous bytes of one row; in the aligned column order its lanes would be 16
-// bytes apart and every line written in four passes (hamming 2000 x 30011 x 166: 300 -> 84 us
-// a call).
+// RAGGED (TX = 64, rows of m % 4 != 0 floats or an unaligned output): rows start at any dword of
+// a line, so a wave takes rows 32 apart, whose starts lie at one place in a 128-byte line, and
+// begins its columns that many floats before the tile's: its 16-byte stores are then aligned and
+// fill whole lines, as the aligned rows' do, but for a row's two ends.  A block takes 8 rows each of
+// 4 of the 32 residues of 256 rows.  (hamming, a call: 16384 x 16383 x 128
+// in 177 us, the aligned 16384 x 16384 160; 2000 x 30011 x 166 in 72.  With 256 contiguous bytes per
+// instruction at each row's own alignment 282 and 84, with dwords in the aligned column order 1279
+// and 299.)
 template <int OP, int EPI, int TX, int CV, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
     const uint32_t *__restrict__ A, const uint32_t *__restrict__ Bw,
@@ -269,12 +272,20 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
     constexpr bool kPops = EPI >= kJaccard;
     constexpr int TY = kThreads / TX, RT = 8 * TY, CT = 8 * TX;
     __shared__ uint4 As[RT][CV + 1];
-    __shared__ uint4 Bs[CT][CV + 1];
+    constexpr int LEAD = RAGGED ? 32 : 0;  // columns staged before the tile's own
+    __shared__ uint4 Bs[CT + LEAD][CV + 1];
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
-    // tile column of the thread's j-th output
-    auto tile_col = [tx](int j) { return RAGGED ? tx + TX * j : (j >> 2) * (4 * TX) + 4 * tx + (j & 3); };
     const int64_t b = blockIdx.z;
-    const int64_t row0 = (int64_t)blockIdx.y * RT, col0 = (int64_t)blockIdx.x * CT;
+    const int64_t row0 = RAGGED ? (int64_t)(blockIdx.y >> 3) * (8 * LEAD) + (blockIdx.y & 7) * TY
+                                : (int64_t)blockIdx.y * RT;
+    const int64_t col0 = (int64_t)blockIdx.x * CT;
+    // row r of As in the output; the thread's row i is row ty + TY i of As
+    auto tile_row = [row0](int r) { return row0 + (RAGGED ? r % TY + LEAD * (r / TY) : r); };
+    int shift = 0;
+    if constexpr (RAGGED)
+        shift = (int)((reinterpret_cast<uintptr_t>(out) / 4 + (uint64_t)(b * n + tile_row(ty)) * (uint64_t)m) % LEAD);
+    // tile column of the thread's j-th output
+    auto tile_col = [tx, shift](int j) { return (j >> 2) * (4 * TX) + 4 * tx + (j & 3) - shift; };
     const uint32_t *Ab = A + b * n * W;
     const uint32_t *Bb = Bw + b * m * W;
 
@@ -288,16 +299,16 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
         const int q = (int)((W - w0) / 4 < CV ? (W - w0) / 4 : CV);
         for (int idx = tid; idx < RT * q; idx += kThreads) {
             const int r = idx / q, c = idx - r * q;
-            const int64_t gr = row0 + r;
+            const int64_t gr = tile_row(r);
             uint4 u = {0u, 0u, 0u, 0u};
             if (gr < n) u = *reinterpret_cast<const uint4 *>(Ab + gr * W + w0 + 4 * c);
             As[r][c] = u;
         }
-        for (int idx = tid; idx < CT * q; idx += kThreads) {
+        for (int idx = tid; idx < (CT + LEAD) * q; idx += kThreads) {
             const int r = idx / q, c = idx - r * q;
-            const int64_t gc = col0 + r;
+            const int64_t gc = col0 + r - LEAD;
             uint4 v = {0u, 0u, 0u, 0u};
-            if (gc < m) v = *reinterpret_cast<const uint4 *>(Bb + gc * W + w0 + 4 * c);
+            if (gc >= 0 && gc < m) v = *reinterpret_cast<const uint4 *>(Bb + gc * W + w0 + 4 * c);
             Bs[r][c] = v;
         }
         __syncthreads();
@@ -306,7 +317,7 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i) a[i] = As[ty + TY * i][c];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bv[j] = Bs[tile_col(j)][c];
+            for (int j = 0; j < 8; ++j) bv[j] = Bs[tile_col(j) + LEAD][c];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -317,40 +328,29 @@ __global__ __launch_bounds__(kThreads) void bool_reduce_kernel(
 
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int64_t row = row0 + ty + TY * i;
+        const int64_t row = tile_row(ty + TY * i);
         if (row >= n) continue;
         float *orow = out + (b * n + row) * m;
         uint32_t pa = 0;
         if constexpr (kPops) pa = (uint32_t)popA[b * n + row];
         const float df = (float)d;
-        if constexpr (RAGGED) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t col = col0 + tile_col(j);
-                uint32_t pb = 0;
-                if constexpr (kPops) pb = col < m ? (uint32_t)popB[b * m + col] : 0u;
-                const float v = finish<OP, EPI>(acc[i][j], pa, pb, (uint32_t)d, inv_d, df, inv_df);
-                if (col < m) orow[col] = v;
-            }
-            continue;
-        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int64_t col = col0 + 4 * TX * h + 4 * tx;
+            const int64_t col = col0 + tile_col(4 * h);
             float v[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 uint32_t pb = 0;
-                if constexpr (kPops) pb = col + c < m ? (uint32_t)popB[b * m + col + c] : 0u;
+                if constexpr (kPops) pb = col + c >= 0 && col + c < m ? (uint32_t)popB[b * m + col + c] : 0u;
                 v[c] = finish<OP, EPI>(acc[i][4 * h + c], pa, pb, (uint32_t)d, inv_d, df, inv_df);
             }
-            if (vec_store && col + 3 < m) {
+            if ((RAGGED || vec_store) && col >= 0 && col + 3 < m) {
                 floatx4 f = {v[0], v[1], v[2], v[3]};
                 store_nt4(orow + col, f);
             } else {
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    if (col + c < m) store_nt(orow + col + c, v[c]);
+                    if (col + c >= 0 && col + c < m) store_nt(orow + col + c, v[c]);
             }
         }
     }
@@ -364,8 +364,10 @@ int launch_reduce(const uint32_t *a, const uint32_t *b, const int32_t *pa, const
     const float inv_df = 1.0f / (float)d;  // as ATen's host-side reciprocal of a CPU scalar
     const bool vec_store = (m % 4 == 0) && aligned16(out);
     const LaunchEvents ev = launch_events("bool_reduce_kernel");
-    if (W <= 8 && m > 256 && cdiv(n, 32) <= kMaxGridYZ) {
-        dim3 grid((unsigned)cdiv(m, 512), (unsigned)cdiv(n, 32), (unsigned)batch);
+    const int64_t grid_y = vec_store ? cdiv(n, 32) : cdiv(n, 256) * 8;
+    if (W <= 8 && m > 256 && grid_y <= kMaxGridYZ) {
+        // ragged: a row's columns begin up to 31 floats before a tile's
+        dim3 grid((unsigned)cdiv(vec_store ? m : m + 31, 512), (unsigned)grid_y, (unsigned)batch);
         if (!vec_store)
             hipExtLaunchKernelGGL((bool_reduce_kernel<OP, EPI, 64, 2, true>), grid, dim3(kThreads), 0, s, ev.start,
                                   ev.stop, 0, a, b, pa, pb, n, m, W, d, inv_d, inv_df, out, vec_store);
