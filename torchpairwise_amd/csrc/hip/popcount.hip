@@ -943,8 +943,10 @@ __global__ __launch_bounds__(tile::kThreads, 4) void bool_fp4_tile_kernel(
 // for pair p of the chunk and feeds word t of it to step t: bit 4 i + e of the word becomes
 // nibble i of operand dword e (0x2 = 1.0 or 0), the same permutation of the features on both
 // sides, so every AND count is unchanged.  A partial last chunk (W % 32 != 0) loads an
-// in-row piece into the slots past the row's end and zeroes them in LDS before use.  Counts, popcounts and the epilogue are those of
-// bool_fp4_tile_kernel, so the outputs are the same bit for bit.  Needs d < 2^24, a 16-byte
+// in-row piece into the slots past the row's end and multiplies only the piece pairs that hold bits,
+// an odd count's last slot zeroed in LDS before use (16384^2 jaccard, a call: 128 features 222 ->
+// 215 us, 700 features 257 -> 254; 900 x 1101 x 1500 32 -> 28).  Counts, popcounts and the epilogue
+// are those of bool_fp4_tile_kernel, so the outputs are the same bit for bit.  Needs d < 2^24, a 16-byte
 // aligned output and rows * W * 4 < 2^32.
 template <int OP, int EPI, bool RAGGED>
 __global__ __launch_bounds__(tile::kThreads, 4) void bool_bits_tile_kernel(
@@ -1036,15 +1038,18 @@ __global__ __launch_bounds__(tile::kThreads, 4) void bool_bits_tile_kernel(
             dma(kc);
         }
         barrier_all();  // chunk kc (and, the first time, the counts) has landed
-        if (kc == nchunks - 1 && vp < 8) {
-            // the partial last chunk: zero the slots past the rows' end (they add nothing)
+        // the partial last chunk: only the piece pairs that hold bits; an odd count's last pair has
+        // a slot past the rows' end, zeroed here (it adds nothing)
+        const int live = kc == nchunks - 1 ? vp : 8;
+        if (live & 1) {
 #pragma unroll
             for (int j = 0; j < kSlots; ++j)
                 if ((bad >> j) & 1) smem[(wave * kSlots + j) * 64 + lane] = make_uint4(0, 0, 0, 0);
             barrier_lds();
         }
 #pragma unroll
-        for (int p = 0; p < 4; ++p) pair(p);
+        for (int p = 0; p < 4; ++p)
+            if (2 * p < live) pair(p);
     }
     const bool small = d <= kSmallRowLimit;
     pops_to_float(small, s_pop);
