@@ -326,10 +326,15 @@ int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch,
                        int64_t n, int64_t m, int64_t d, const float *aux1,
                        const float *aux2, int epilogue, void *out, void *stream);
 
+/* tpw_pairwise_inner without norm arrays: the small-output kernel forms them itself (one launch,
+ * the same bits as with tpw_row_norms' arrays).  TPW_ERR_INVALID where
+ * tpw_pairwise_inner_forms_norms is 0 and the epilogue uses norms. */
+int tpw_pairwise_inner_own_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
+                                 int64_t m, int64_t d, int epilogue, void *out, void *stream);
+
 /* 1 where tpw_pairwise_inner runs its small-output kernel on these operands (only the alignment
- * of x1 and x2 is looked at), which takes rows of any length and
- * alignment at full speed and, when aux1 and aux2 are both NULL, forms the norms itself (one
- * launch, the same bits as with tpw_row_norms' arrays); else 0: there the norms are required.  Replaces no reference kernel (its norms are separate ATen calls). */
+ * of x1 and x2 is looked at), which takes rows of any length and alignment at full speed; else 0.
+ * Replaces no reference kernel (its norms are separate ATen calls). */
 int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch,
                                    int64_t n, int64_t m, int64_t d);
 

@@ -104,7 +104,7 @@ def test_small_output_kernel_equals_tile_kernels(dtype, n, m, d, epi):
         own = torch.empty((1, n, m), dtype=dtype, device=DEV)
         a, c = x1[b].clone(), x2[b].clone()
         assert small(a, c, 1)
-        capi.call("tpw_pairwise_inner", capi._ptr(a), capi._ptr(c), capi._dtype_code(a), 1, n, m, d, None, None, epi,
+        capi.call("tpw_pairwise_inner_own_norms", capi._ptr(a), capi._ptr(c), capi._dtype_code(a), 1, n, m, d, epi,
                   capi._ptr(own), capi._stream())
         assert _same_bits(own, given)
         if dtype == torch.bfloat16 and epi >= capi.EPI_COSINE_SIM:

@@ -26,6 +26,9 @@
 //   4. finalize: one wave per pair rescans the winning m for the first n position reaching
 //      its min, and writes sqrt, and the (permuted) indices.
 //
+// Small clouds (use_dense) skip all of it: dense_kernel evaluates every point pair and
+// dense_finish_kernel picks the result, two launches where the grid takes ten.
+//
 // Non-negative fp32 bit patterns order like the values, so the packed key orders by
 // (value, m position) exactly.  That argument needs finite coordinates: with a NaN or an
 // infinity the loop's updates depend on the order of the NaN sums (a row whose last sum is NaN

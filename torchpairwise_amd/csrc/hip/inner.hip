@@ -19,6 +19,8 @@
 //     whose outputs are not stored).  120 VGPRs: 4 waves per SIMD, 4 blocks per CU;
 //   register prefetch (any d): the next chunk's global loads are issued into registers
 //     before the current chunk's MFMAs, and stored to LDS after them (zero padding past d).
+// Outputs of few tiles (small_fits) take inner_small_kernel: 64 x 64 tiles, rows of any length and
+// alignment, the norms formed from the staged rows, so that the call is one launch.
 // Tiles are assigned XCD-contiguously (consecutive workgroup ids go round-robin over the
 // 8 XCDs, so id % 8 selects the XCD) and in groups of 8 tile rows, so that the blocks
 // resident on one XCD share A and B panels in that XCD's L2.
@@ -1502,9 +1504,11 @@ extern "C" int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, in
                : 0;
 }
 
-extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch,
-                                  int64_t n, int64_t m, int64_t d, const float *aux1,
-                                  const float *aux2, int epilogue, void *out, void *stream) {
+namespace {
+
+// Both entries below; own_norms: aux1 and aux2 null, formed by the small-output kernel.
+int run_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n, int64_t m, int64_t d,
+                       const float *aux1, const float *aux2, bool own_norms, int epilogue, void *out, void *stream) {
     TPW_REQUIRE(dtype == TPW_F32 || dtype == TPW_BF16, "unsupported dtype %d", dtype);
     TPW_REQUIRE(epilogue >= TPW_EPI_DOT && epilogue <= TPW_EPI_CORRELATION, "unknown epilogue %d",
                 epilogue);
@@ -1512,7 +1516,7 @@ extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int
     if (batch == 0 || n == 0 || m == 0) return TPW_OK;
     TPW_REQUIRE(x1 && x2 && out, "null pointer");
     TPW_REQUIRE(epilogue == TPW_EPI_DOT || (aux1 && aux2) ||
-                    (!aux1 && !aux2 && tpw_pairwise_inner_forms_norms(x1, x2, dtype, batch, n, m, d)),
+                    (own_norms && tpw_pairwise_inner_forms_norms(x1, x2, dtype, batch, n, m, d)),
                 "norms required for epilogue %d", epilogue);
     const int64_t total = cdiv(n, kTile) * cdiv(m, kTile) * batch;
     TPW_REQUIRE(total <= 0x7fffffffLL, "output too large for one launch");
@@ -1523,6 +1527,19 @@ extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int
     return dispatch_epi<uint16_t>(static_cast<const uint16_t *>(x1),
                                   static_cast<const uint16_t *>(x2), batch, n, m, d, aux1, aux2,
                                   epilogue, static_cast<uint16_t *>(out), s);
+}
+
+}  // namespace
+
+extern "C" int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch,
+                                  int64_t n, int64_t m, int64_t d, const float *aux1,
+                                  const float *aux2, int epilogue, void *out, void *stream) {
+    return run_pairwise_inner(x1, x2, dtype, batch, n, m, d, aux1, aux2, false, epilogue, out, stream);
+}
+
+extern "C" int tpw_pairwise_inner_own_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
+                                            int64_t m, int64_t d, int epilogue, void *out, void *stream) {
+    return run_pairwise_inner(x1, x2, dtype, batch, n, m, d, nullptr, nullptr, true, epilogue, out, stream);
 }
 
 extern "C" int tpw_radius_mask_euclidean(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,

@@ -34,6 +34,9 @@
 //         grad_x2) k-major through transposing LDS reads (grad_product_bf16); other shapes
 //         write W^T and transposed x1, x2 so that both products are A . B^T with k-contiguous
 //         rows (inner_grad_gemm).
+// Small and middle problems (op_fits) take neither: op_backward_kernel forms the weights while
+// staging and runs both gradients' products in one launch, split over the sums where the tiles
+// leave CUs idle, and op_finish_kernel adds the splits and the coefficients.
 #include <type_traits>
 
 #include "common.hpp"

@@ -12,7 +12,7 @@
 // pair more for general p.  Stores are non-temporal float4 rows (256 B per 16 lanes).
 // Bray-Curtis runs the p = 1 kernel for sum |a - b| and a second pass for sum |a + b| that
 // divides the stored numerator (two accumulators per output would halve the register
-// tile; the VALU work is the same).
+// tile; the VALU work is the same).  Grids that leave CUs idle take 64 x 64 tiles instead.
 //
 // Backward (grad of x1; x2 by the transposed call): out[i,k] = sum_j F(x1[i,k], x2[j,k],
 // per-pair weights of (i, j)).  A block owns 128 rows x 64 features with its x1 values held
@@ -20,7 +20,8 @@
 // computed while staging into LDS), thread block 8 rows x 4 features.  The j range is
 // split over several blocks when the row/feature grid alone would not fill the GPU; the
 // per-split partial sums are then added in split order by a second kernel, so the result
-// is deterministic (the reference accumulates with atomics on its GPU path).
+// is deterministic (the reference accumulates with atomics on its GPU path).  Above 64 features
+// p = 2, 3 and general p > 2 (and p = 1 where its range scan allows) own 128 features a block.
 #include <math.h>
 
 #include <type_traits>

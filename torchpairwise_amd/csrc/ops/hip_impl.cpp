@@ -129,10 +129,12 @@ at::Tensor pw_inner_cuda(const at::Tensor &x1, const at::Tensor &x2, int64_t epi
             bp.narrow(2, 0, d).copy_(b);
         }
     }
-    check_rc(tpw_pairwise_inner(ap.data_ptr(), bp.data_ptr(), dt, B, n, m, dk,
-                                n1.defined() ? n1.data_ptr<float>() : nullptr,
-                                n2.defined() ? n2.data_ptr<float>() : nullptr, (int)epilogue,
-                                out.data_ptr(), s),
+    check_rc(small ? tpw_pairwise_inner_own_norms(a.data_ptr(), b.data_ptr(), dt, B, n, m, d, (int)epilogue,
+                                                  out.data_ptr(), s)
+                   : tpw_pairwise_inner(ap.data_ptr(), bp.data_ptr(), dt, B, n, m, dk,
+                                        n1.defined() ? n1.data_ptr<float>() : nullptr,
+                                        n2.defined() ? n2.data_ptr<float>() : nullptr, (int)epilogue,
+                                        out.data_ptr(), s),
              "_pw_inner");
     return out_shape(out, x1);
 }
