@@ -237,12 +237,12 @@ def test_backward_products_tile_fp32(name, kw, B, n, m, d):
 
 
 # Both gradients in one launch (op_backward_kernel): edges of its 64-row tiles, 64- and 128-feature
-# tiles, 32-row K chunks and splits, sums long enough to be blocked (512), vector and element
+# tiles, 32-row K chunks and splits (also of one direction alone), sums long enough to be blocked (512), vector and element
 # loads; a zero row (norm 0) and rows out of the fast cosine terms' norm range.  fp32 against the
 # derived per-element bounds (euclidean, cosine) or, like the kernel functions above, rtol 1e-4;
 # bf16 at the bf16 tolerance of the other paths.
 @pytest.mark.parametrize("B,n,m,d", [(1, 1, 1, 1), (1, 63, 65, 64), (2, 65, 33, 65), (1, 31, 1100, 30),
-                                     (1, 1601, 64, 128), (3, 130, 97, 131)])
+                                     (1, 1601, 64, 128), (3, 130, 97, 131), (4, 9000, 40, 130)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("name,kw", [o for o in BWD_OPS if o[0] != "polynomial_kernel"])
 def test_backward_one_launch(name, kw, dtype, B, n, m, d):

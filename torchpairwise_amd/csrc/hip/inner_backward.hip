@@ -817,6 +817,12 @@ OpPlan op_plan(int64_t batch, int64_t n, int64_t m, int64_t d) {
     const int64_t rows[2] = {n, m};
     const int64_t base = (cdiv(n, kOpRows) + cdiv(m, kOpRows)) * P.tiles_f * batch;
     const int64_t fill = 2 * device_cus();
+    // Chunks of the whole launch per block slot.  Where n and m are far apart the many blocks of
+    // one direction fill the chip and the few of the other would each walk the long K alone
+    // (8 x 100 x 12001 x 150, euclidean forward and backward: 1268 -> 383 us), so a
+    // block takes at most one and a half shares, and eight chunks without asking.
+    const int64_t share =
+        (cdiv(n, kOpRows) * cdiv(m, kOpK) + cdiv(m, kOpRows) * cdiv(n, kOpK)) * P.tiles_f * batch * 3 / (2 * fill);
     for (int t = 0; t < 2; ++t) {
         OpDir &D = P.dir[t];
         D.R = rows[t];
@@ -826,6 +832,8 @@ OpPlan op_plan(int64_t batch, int64_t n, int64_t m, int64_t d) {
         // the longer K takes more of the splits: its blocks are the longer ones
         const int64_t longer = n > m ? n : m;
         sp = cdiv(sp * D.K, longer < 1 ? 1 : longer);
+        const int64_t even = cdiv(cdiv(D.K, kOpK), share < 8 ? 8 : share);
+        sp = even > sp ? even : sp;
         sp = sp > 32 ? 32 : sp < 1 ? 1 : sp;
         D.kps = cdiv(cdiv(D.K, sp), kOpK) * kOpK;
         D.splits = D.K > 0 ? cdiv(D.K, D.kps) : 1;
