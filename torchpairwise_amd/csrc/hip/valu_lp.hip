@@ -695,7 +695,8 @@ __global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
     // or past jend only reach accumulators of rows, features or stage steps that are never stored
     // or run.  Dword loads throughout cost the narrow
     // kernel 12 more load instructions per stage, and held the wide one to n, m and d that are
-    // multiples of 4 (rbf 4096 x 4000 x 90, the narrow kernel before: backward 409 -> 230 us).
+    // multiples of 4 (rbf 4096 x 4000 x 90, forward and backward, the
+    // narrow kernel before: 442 -> 309 us).
     constexpr bool kReadG = !PRE;                               // upstream grad
     constexpr bool kReadA0 = PRE || (MODE == kRoot && PK != kP1);  // weights, or the distance
     constexpr bool kReadA1 = PRE && kTwo;
