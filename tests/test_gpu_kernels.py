@@ -616,6 +616,21 @@ def test_hausdorff_grid_above_dense_bit_exact(case):
     _hd_check(x1, x2, perm1, perm2, case)
 
 
+# Which calls evaluate every point pair (two launches): those that cost less so than the grid's
+# passes.  Many pairs of clouds, or few blocks with a long x2, stay on the grid.
+@pytest.mark.parametrize("clouds,p1,p2,d,dense", [
+    (64, 2896, 2896, 3, False), (64, 2896, 2896, 1, False), (64, 256, 32768, 3, False), (64, 256, 32768, 2, False),
+    (64, 2048, 1024, 2, False), (100, 333, 3000, 3, False), (16, 2896, 2896, 2, False), (1, 64, 32768, 3, False),
+    (1, 256, 32768, 2, False), (1, 8000, 8000, 3, True), (16, 1024, 1024, 2, True), (64, 724, 724, 3, True),
+    (4, 32768, 256, 1, True), (200, 100, 100, 3, True), (1, 64, 32768, 1, True),
+])
+def test_hausdorff_dense_where_cheaper(clouds, p1, p2, d, dense):
+    x1, x2 = (t.to(DEV) for t in _hd_inputs(None, clouds, p1, clouds, p2, d, seed=70))
+    c = capi.HausdorffCounters().arm()
+    capi.directed_hausdorff(x1, x2)
+    assert (c.read()["launches"] == 2) == dense
+
+
 def test_hausdorff_counters():
     """The work counters: the kernels evaluate far fewer pairs than brute force, the sorted
     mode's cell scan runs its box tests, the forward of a few clouds is ten launches, and

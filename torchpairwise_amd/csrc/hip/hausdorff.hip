@@ -2446,15 +2446,42 @@ int launch_dense(int64_t pairs, void *ws, const float *x1, const float *x2, int6
     return check_launch("hausdorff dense");
 }
 
-// Which calls it takes.  It evaluates 5.4e12 pairs a second; the grid costs 70 us for one pair of
-// clouds, and 3 us a pair of clouds at 1000 to 2000 points (few points per cell), 1.6 at 4100.
-// Measured, grid -> dense: 1 x 1 clouds of 8000 points 89 -> 32 us, 16300 79 -> 57 (2^28 point
-// pairs; 30000: 74, against 167 at that rate); 8 x 8 of 512 475 -> 14, 16 x 16 of 1020 715 -> 58;
-// 16 x 16 of 4100 stays on the grid (412 us against 797).  The finish scans x2 by one block per
+// Which calls it takes: those whose every pair costs less than the least that the grid was seen to
+// take, on uniform clouds of 4 to 32768 points, 1 x 1 to 200 x 200 of them.  Microseconds.
+// Dense: blocks of 64 m at 0.2 ns a wave and 3, 6.2 or 9 ns a thousand points of x2 (d = 1, 2, 3;
+// 64 x 64 clouds of 2048 points 1240 / 1960 / 2730 us), and no less than the chain of one block
+// over x2 (1 x 1 of 64 x 32768 points 42 / 69 / 101 us).
+inline double dense_cost(int64_t d, int64_t pairs, int64_t p1, int64_t p2) {
+    const double wave = d == 1 ? 0.25e-3 : 0.2e-3, point = d == 1 ? 0.003e-3 : d == 2 ? 0.0062e-3 : 0.009e-3;
+    const double chain = d == 1 ? 0.9e-3 : d == 2 ? 1.7e-3 : 2.7e-3;
+    const double block = wave * dense_waves(p2) + point * (double)p2;
+    return 13.0 + std::max(chain * (double)p2, (double)(pairs * cdiv(p1, 64)) * block);
+}
+// Grid: its chain of launches, which the x1 points (up to some 1500 a cloud) lengthen while x2 has
+// few points per cell, and its share per pair of clouds.  (64 x 64 clouds: 2048 points 1230 / 560 /
+// 1560 us, 256 x 32768 points 1152 / 395 / 419; 16 x 16 of 2048 290 / 197 / 790.)  Where x2 has few
+// points and x1 four times as many, ball queries walk mostly empty rings: several times that.
+inline double grid_cost(int64_t d, int64_t pairs, int64_t p1, int64_t p2) {
+    const double n = (double)pairs, m = (double)std::min<int64_t>(p1, 1500);
+    if (d == 1) return 240.0 + n * (p2 <= 64 ? 1.6 : p2 <= 128 ? 0.45 : 0.2);
+    const bool few = p1 >= 4 * p2 && p2 <= 512;
+    if (d == 2) {
+        const double g = p2 >= 4096 ? 58.0 + 0.075 * n : 55.0 + 0.07 * m + 0.085 * n;
+        return few ? std::max(g, 400.0 + n * (p2 <= 128 ? 0.8 : p2 <= 256 ? 0.45 : 0.2)) : g;
+    }
+    const double g = p2 >= 8192   ? 60.0 + 0.08 * n
+                     : p2 >= 4096 ? 60.0 + 0.2 * m + 0.08 * n
+                                  : 50.0 + 0.32 * m + (0.09 + 0.00007 * m) * n;
+    return few ? std::max(g, 700.0 + n * (p2 <= 128 ? 0.85 : p2 <= 256 ? 0.55 : 0.4)) : g;
+}
+// Grid -> dense, d = 3: 1 x 1 clouds of 8000 points 119 -> 33 us, 16 x 16 of 1024 705 -> 58, 64 x 64
+// of 1024 1442 -> 836; these stay on the grid: 64 x 64 of 2896 (1295 against 5210), of 256 x 32768
+// (418 against 4860), 1 x 1 of 64 x 32768 (63 against 101).  The finish scans x2 by one block per
 // pair of clouds, hence the limit on points; a launch holds fewer than 2^32 threads.
-inline bool use_dense(int64_t pairs, int64_t p1, int64_t p2) {
+inline bool use_dense(int64_t d, int64_t pairs, int64_t p1, int64_t p2) {
     return p1 <= 32768 && p2 <= 32768 && pairs * cdiv(p1, 64) * 64 * dense_waves(p2) < ((int64_t)1 << 31) &&
-           (p1 * p2 <= ((int64_t)1 << 23) || pairs * p1 * p2 <= ((int64_t)1 << 28));
+           (p1 * p2 <= ((int64_t)1 << 23) || pairs * p1 * p2 <= ((int64_t)1 << 28)) &&
+           dense_cost(d, pairs, p1, p2) <= grid_cost(d, pairs, p1, p2);
 }
 
 // Counting sort into records: x2's clouds (sets S2), then, when S1 has clouds, x1's; cell starts
@@ -2637,7 +2664,7 @@ extern "C" int tpw_directed_hausdorff(const float *x1, const float *x2, int64_t 
     hipStream_t s = as_stream(stream);
     const Plan P = make_plan(batch, b1, p1, b2, p2, d);
     const Workspace w = carve(workspace, P, p1, p2, d);
-    if (P.sorted && use_dense(pairs, p1, p2)) {
+    if (P.sorted && use_dense(d, pairs, p1, p2)) {
         switch (d) {
             case 1: return launch_dense<1>(pairs, workspace, x1, x2, b1, p1, b2, p2, perm1, perm2, out, idx1, idx2, s);
             case 2: return launch_dense<2>(pairs, workspace, x1, x2, b1, p1, b2, p2, perm1, perm2, out, idx1, idx2, s);
