@@ -39,6 +39,14 @@ def test_pure_host_entry_points():
     assert l.tpw_hausdorff_workspace_size(1, 2, 10, 3, 20, 3) > 0
 
 
+def test_hausdorff_workspace_fits_the_static_buffer():
+    # regression: sized for the dense kernels' keys where those never run (pairs x p1 > 2^28), which
+    # the allocation-free entry then refused: 101, 155 and 119 MiB
+    l = _capi.lib()
+    for sizes in ((1, 255, 13000, 255, 1000, 3), (1, 255, 20000, 255, 200, 2), (1, 200, 25000, 200, 500, 1)):
+        assert l.tpw_hausdorff_workspace_size(*sizes) <= 96 << 20, sizes
+
+
 def test_argument_errors_are_reported_without_gpu():
     l = _capi.lib()
     # invalid sizes are rejected on the host before any launch

@@ -2611,9 +2611,11 @@ extern "C" size_t tpw_hausdorff_workspace_size(int64_t batch, int64_t b1, int64_
                                                int64_t p2, int64_t d) {
     if (batch < 0 || b1 < 0 || b2 < 0 || p1 < 0 || p2 < 0 || d < 0) return 0;
     size_t total = 0;
+    // The dense kernels' keys (8 bytes per pair and 64 m) lie over the grid's arrays: they run in
+    // the sorted mode alone, whose keys (8 bytes per pair) and flag bits (4 bytes per pair and 32 m)
+    // are at least as long.
     carve(nullptr, make_plan(batch, b1, p1, b2, p2, d), p1, p2, d, &total);
-    // the dense kernels' keys (8 bytes per pair and 64 m) lie over the grid's arrays
-    return std::max<size_t>(total, align256(8 * (size_t)(batch * b1 * b2) * (size_t)cdiv(p1, 64)));
+    return total;
 }
 
 extern "C" int tpw_hausdorff_counters(int arm, unsigned long long *out) {
