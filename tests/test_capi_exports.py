@@ -47,6 +47,31 @@ def test_hausdorff_workspace_fits_the_static_buffer():
         assert l.tpw_hausdorff_workspace_size(*sizes) <= 96 << 20, sizes
 
 
+def test_small_output_rule():
+    """Where the 64 x 64 inner-product kernel runs (256 CUs): not where the 128 x 128 tile kernel,
+    padded copies or not, takes less (regression: wide rows went there, up to 2.2 times as slow)."""
+    l = _capi.lib()
+
+    def small(dtype, b, n, m, d, offset=0):
+        return bool(l.tpw_pairwise_inner_forms_norms(4096 + offset, 8192, dtype, b, n, m, d))
+
+    f32, bf16 = 0, 1
+    for d in (256, 512, 1000, 1024, 2048):  # ragged m and partial chunks at 256 tiles
+        assert not small(f32, 1, 2048, 2047, d) and not small(f32, 1, 2000, 2047, d)
+        if d >= 1000:
+            assert not small(bf16, 1, 2048, 2048, d) and not small(bf16, 1, 2000, 2047, d)
+    assert not small(f32, 1, 2048, 2048, 500) and not small(f32, 1, 1664, 2048, 500)
+    assert not small(f32, 1, 1700, 1999, 512) and not small(f32, 1, 1280, 2048, 768)
+    for d in (1024, 2048, 4096, 65536):  # bf16 rows of whole chunks
+        assert not small(bf16, 1, 1024, 2048, d) and not small(bf16, 1, 300, 5000, d)
+        assert not small(bf16, 1, 64, 64, d)
+    for n, m, d in ((64, 64, 128), (37, 1003, 50), (1000, 1000, 4096), (1024, 2048, 1000), (1280, 2041, 128)):
+        assert small(f32, 1, n, m, d) and small(bf16, 1, n, m, min(d, 500))
+        assert small(f32, 1, n, m, d, 4) and small(bf16, 1, n, m, min(d, 500), 2)
+    assert small(f32, 250, 128, 128, 1000) and small(bf16, 250, 128, 128, 3000) and small(bf16, 1, 16000, 60, 768)
+    assert not small(f32, 260, 64, 64, 50) and not small(bf16, 260, 64, 64, 50)
+
+
 def test_argument_errors_are_reported_without_gpu():
     l = _capi.lib()
     # invalid sizes are rejected on the host before any launch

@@ -1051,17 +1051,32 @@ int64_t cu_count() {
     return c;
 }
 
-// Whether the small kernel takes the call: up to half as many 128 x 128 tiles as CUs, or as many
-// where the tile kernel would need padded copies of the operands or the staged kernel would run
-// (rows that are no whole aligned chunks, fp32 rows of m % 4 != 0 outputs).  Whole call, norms
-// launched -> formed inside: fp32 37 x 1003 x 50 15.3 -> 6.8 us, 700 x 900 x 128 17.5 -> 8.9, 8 x
-// 227 x 544 x 224 26.7 -> 16.8; bf16 1501 x 999 x 100 34.8 -> 10.2; at 144 tiles of d = 512 42.6
-// -> 41.9; at 256 tiles of whole chunks the tile kernel stays ahead (2048^2: d = 128 20.2 against
-// 23.1, d = 512 43.4 against 69.4), ragged 2047 x 2041 x 101 34.9 -> 23.8.
+// Whether the small kernel takes the call: at most as many 128 x 128 tiles as CUs, and its own
+// blocks no dearer than what the rows would take otherwise.  All times are of whole calls, others -> small.
+// Rows of whole aligned chunks would take the tile kernel behind a norm launch.  fp32: up to two
+// blocks a CU at any d (37 x 1003 x 128 15.6 -> 8.4 us, 1024 x 2048 x 4096 267 -> 240), up to three
+// to d = 384 (1280 x 2048: d = 256 24.2 -> 22.9, but 512 39.3 -> 40.4 and 2048 137 -> 154; 2048^2 x 512,
+// four a CU, 40.6 -> 68).  bf16's chunks are a fifth as dear there: to d = 256 and 512 (1024 x 2048: d =
+// 256 10.4 -> 8.7, 512 11.4 -> 12.4 with a launch less, 1024 15.1 -> 20.2, 2048 26 -> 36), and 896 where
+// the norm pass reads many rows (16000 x 60 x 768 21.8 -> 15.9, 2376 x 32 in 4 batches x 896 19.8 -> 16.7).
+// Other rows would be copied zero-padded first, from 2^20 outputs on (fp32 1280 x 2048 x 1000 90 -> 80;
+// bf16 1024 x 2048 x 1500 46 -> 30, but x 3000 58 -> 65), or take the staged kernel, four times as
+// slow by elements (bf16 1000^2 x 500 44 -> 14) as by 16-byte pieces (1000^2 x 1000 23 -> 20, x 3000
+// 56 -> 64).  Four blocks a CU pay at few features (2048^2: fp32 d = 300 45.9 -> 44.1, 500 58 -> 69;
+// bf16 500 27.6 -> 27.3, 1000 35.6 -> 39.4) or where the copies are of many rows (250 x 128 x 128
+// fp32 x 1000 248 -> 179, bf16 106 -> 50).
 template <typename T>
 bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d) {
-    const bool whole = d % Elem<T>::kChunk == 0 && aligned16(x1) && aligned16(x2) && (sizeof(T) == 2 || m % 4 == 0);
-    return cdiv(n, kTile) * cdiv(m, kTile) * batch * (whole ? 2 : 1) <= cu_count();
+    const int64_t cus = cu_count(), blocks = cdiv(n, kST) * cdiv(m, kST) * batch, rows = batch * (n + m);
+    if (cdiv(n, kTile) * cdiv(m, kTile) * batch > cus) return false;
+    constexpr bool f32 = sizeof(T) == 4;
+    const bool row16 = d % Elem<T>::kPer16 == 0 && aligned16(x1) && aligned16(x2);
+    const bool two = blocks <= 2 * cus, three = blocks <= 3 * cus;
+    if (row16 && d % Elem<T>::kChunk == 0)
+        return f32 ? two || (three && d <= 384) : (three && d <= 256) || (two && d <= (rows >= 8192 ? 896 : 512));
+    if (!row16 && batch * n * m < ((int64_t)1 << 20)) return true;
+    if (f32) return three || d <= 320 || rows >= 16384 + 8 * d;
+    return three ? d <= 2048 || rows >= 8192 : d <= 704 || rows >= 16384;
 }
 
 template <typename T, int EPI>
