@@ -1058,7 +1058,9 @@ int64_t cu_count() {
 // to d = 384 (1280 x 2048: d = 256 24.2 -> 22.9, but 512 39.3 -> 40.4 and 2048 137 -> 154; 2048^2 x 512,
 // four a CU, 40.6 -> 68).  bf16's chunks are a fifth as dear there: to d = 256 and 512 (1024 x 2048: d =
 // 256 10.4 -> 8.7, 512 11.4 -> 12.4 with a launch less, 1024 15.1 -> 20.2, 2048 26 -> 36), and 896 where
-// the norm pass reads many rows (16000 x 60 x 768 21.8 -> 15.9, 2376 x 32 in 4 batches x 896 19.8 -> 16.7).
+// the norm pass reads many rows (16000 x 60 x 768 21.8 -> 15.9, 2376 x 32 in 4 batches x 896 19.8 -> 16.7),
+// 1024 where output rows are no whole 16-byte units (1001 x 999 x 1024 16.4 -> 19.8 in a queue of calls,
+// but 32 -> 33 each alone).
 // Other rows would be copied zero-padded first, from 2^20 outputs on (fp32 1280 x 2048 x 1000 90 -> 80;
 // bf16 1024 x 2048 x 1500 46 -> 30, but x 3000 58 -> 65), or take the staged kernel, four times as
 // slow by elements (bf16 1000^2 x 500 44 -> 14) as by 16-byte pieces (1000^2 x 1000 23 -> 20, x 3000
@@ -1072,8 +1074,11 @@ bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, i
     constexpr bool f32 = sizeof(T) == 4;
     const bool row16 = d % Elem<T>::kPer16 == 0 && aligned16(x1) && aligned16(x2);
     const bool two = blocks <= 2 * cus, three = blocks <= 3 * cus;
-    if (row16 && d % Elem<T>::kChunk == 0)
-        return f32 ? two || (three && d <= 384) : (three && d <= 256) || (two && d <= (rows >= 8192 ? 896 : 512));
+    if (row16 && d % Elem<T>::kChunk == 0) {
+        if (f32) return two || (three && d <= 384);
+        const int64_t most = rows >= 8192 ? 896 : blocks <= cus && m % 8 != 0 ? 1024 : 512;
+        return (three && d <= 256) || (two && d <= most);
+    }
     if (!row16 && batch * n * m < ((int64_t)1 << 20)) return true;
     if (f32) return three || d <= 320 || rows >= 16384 + 8 * d;
     return three ? d <= 2048 || rows >= 8192 : d <= 704 || rows >= 16384;
