@@ -55,12 +55,15 @@ const char *tpw_last_error(void);
 int tpw_runtime_version(void);
 
 /* Launch timer (measurement support; no counterpart in the reference).  Arms HIP event
- * pairs around every launch of one kernel family ("inner_tile_kernel",
- * "pairwise_inner_kernel", "lp_forward_kernel", "bool_reduce_kernel",
- * "bool_bits_tile_kernel") made on the current device, at most `capacity` launches (later ones
+ * pairs around every launch of one kernel family made on the current device, at most `capacity`
+ * launches (later ones
  * are counted as dropped).  Events are recorded on the stream each launch goes to, so a caller
  * reads the device duration of the launches inside its own timed loop.  Creates events the
- * first time (no device memory).  Not for concurrent use from several threads. */
+ * first time (no device memory).  Not for concurrent use from several threads.
+ * Families: "inner_tile_kernel" (the small-output kernel's launches too), "inner_small_kernel"
+ * (those alone), "pairwise_inner_kernel", "lp_forward_kernel", "bool_reduce_kernel",
+ * "bool_reduce_ragged_kernel" (of those, the ragged rows stored in aligned lines),
+ * "bool_bits_tile_kernel", "op_backward_kernel", "grad_wide_bf16_kernel". */
 int tpw_launch_timer_arm(const char *family, int capacity);
 /* Disarms the timer, waits for the recorded events and writes the first min(count,
  * capacity) launch durations in ms to ms[]; *count = launches recorded, *dropped (may be

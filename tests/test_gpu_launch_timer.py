@@ -44,3 +44,17 @@ def test_launch_timer_counts_launches_past_its_capacity():
     torch.cuda.synchronize()
     ms, dropped = timer.read()
     assert len(ms) == 2 and dropped == 3 and all(v > 0 for v in ms)
+
+
+def test_launch_timer_tells_the_small_output_kernel():
+    """The small-output kernel has a name of its own; the tile family counts it too."""
+    def count(family, *sizes):
+        timer = capi.LaunchTimer(family, 8).arm()
+        for n, m in sizes:
+            capi.pairwise_inner(x1[:n], x2[:m], capi.EPI_DOT)
+        torch.cuda.synchronize()
+        return len(timer.read()[0])
+
+    x1, x2 = randn(4096, 64, seed=0).cuda(), randn(4096, 64, seed=1).cuda()
+    assert count("inner_small_kernel", (100, 100), (4096, 4096), (64, 200)) == 2
+    assert count("inner_tile_kernel", (100, 100), (4096, 4096)) == 2

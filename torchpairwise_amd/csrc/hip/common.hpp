@@ -17,12 +17,12 @@ int check_launch(const char *what);
 
 // Start / stop events for one kernel launch (hipExtLaunchKernelGGL stamps them as part of the
 // dispatch, so they add no packets of their own): a free event pair of the launch timer when
-// tpw_launch_timer_arm armed it for this kernel family on the current device, else null events
-// (a plain launch).  launch_timer.hip.
+// tpw_launch_timer_arm armed it for this kernel, or for a family that counts it too, on the current
+// device, else null events (a plain launch).  launch_timer.hip.
 struct LaunchEvents {
     hipEvent_t start = nullptr, stop = nullptr;
 };
-LaunchEvents launch_events(const char *family);
+LaunchEvents launch_events(const char *kernel, const char *family = nullptr);
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

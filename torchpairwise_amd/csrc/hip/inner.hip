@@ -1088,7 +1088,7 @@ template <typename T, int EPI>
 int launch_small(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d, const float *aux1,
                  const float *aux2, T *out, hipStream_t s) {
     const int64_t tiles_n = cdiv(n, kST), tiles_m = cdiv(m, kST), total = tiles_n * tiles_m * batch;
-    const LaunchEvents ev = launch_events("inner_tile_kernel");
+    const LaunchEvents ev = launch_events("inner_small_kernel", "inner_tile_kernel");
     if (kAux1<EPI> && !aux1)
         hipExtLaunchKernelGGL((inner_small_kernel<T, EPI, true>), dim3((unsigned)total), dim3(kThreads), 0, s, ev.start,
                               ev.stop, 0, x1, x2, n, m, d, norm_lanes(x1, d) != 0, norm_lanes(x2, d) != 0, aux1, aux2, out,

@@ -2025,12 +2025,13 @@ int run_op_backward(const OpPlan &P, const T *g, const T *x1, const T *x2, const
     float *p1 = P.finish ? ws + P.part[0] : nullptr, *c1 = P.finish ? ws + P.coef[0] : nullptr;
     float *p2 = P.finish ? ws + P.part[1] : nullptr, *c2 = P.finish ? ws + P.coef[1] : nullptr;
     const dim3 grid((unsigned)(P.dir[0].blocks + P.dir[1].blocks));
+    const LaunchEvents ev = launch_events("op_backward_kernel");
     if (d <= 64)
-        hipLaunchKernelGGL((op_backward_kernel<T, MODE, 64>), grid, dim3(256), 0, s, g, res, x1, x2, n1, n2, n, m, d,
-                           P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
+        hipExtLaunchKernelGGL((op_backward_kernel<T, MODE, 64>), grid, dim3(256), 0, s, ev.start, ev.stop, 0, g, res, x1,
+                              x2, n1, n2, n, m, d, P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
     else
-        hipLaunchKernelGGL((op_backward_kernel<T, MODE, 128>), grid, dim3(256), 0, s, g, res, x1, x2, n1, n2, n, m, d,
-                           P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
+        hipExtLaunchKernelGGL((op_backward_kernel<T, MODE, 128>), grid, dim3(256), 0, s, ev.start, ev.stop, 0, g, res, x1,
+                              x2, n1, n2, n, m, d, P.dir[0], P.dir[1], P.tiles_f, kp, sign, gx1, gx2, p1, c1, p2, c2);
     const int rc = check_launch("op_backward_kernel");
     if (rc != TPW_OK || !P.finish) return rc;
     hipLaunchKernelGGL(op_finish_kernel<T>, dim3((unsigned)cdiv(batch * (n + m) * d, 256)), dim3(256), 0, s, p1, c1,

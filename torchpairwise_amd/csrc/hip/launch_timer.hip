@@ -29,11 +29,12 @@ std::atomic<int> g_armed{0};
 
 }  // namespace
 
-LaunchEvents launch_events(const char *family) {
+LaunchEvents launch_events(const char *kernel, const char *family) {
     LaunchEvents e;
     if (!g_armed.load(std::memory_order_relaxed)) return e;
     std::lock_guard<std::mutex> lk(g_timer.mu);
-    if (!g_armed.load(std::memory_order_relaxed) || strcmp(family, g_timer.family) != 0) return e;
+    if (!g_armed.load(std::memory_order_relaxed)) return e;
+    if (strcmp(kernel, g_timer.family) != 0 && (!family || strcmp(family, g_timer.family) != 0)) return e;
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev != g_timer.device) return e;
     if (g_timer.used >= g_timer.capacity) {
