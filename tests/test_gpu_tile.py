@@ -17,6 +17,21 @@ from torchpairwise_amd import _capi as capi
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
+
+class Launches:
+    """The launches of one kernel family inside a ``with`` block: which path a call took."""
+
+    def __init__(self, family):
+        self.timer = capi.LaunchTimer(family, 16)
+
+    def __enter__(self):
+        self.timer.arm()
+        return self
+
+    def __exit__(self, *exc):
+        self.count = len(self.timer.read()[0])
+
+
 EPIS = [capi.EPI_DOT, capi.EPI_EUCLIDEAN, capi.EPI_SQEUCLIDEAN, capi.EPI_COSINE_SIM,
         capi.EPI_COSINE_DIST, capi.EPI_CORRELATION]
 
@@ -186,6 +201,22 @@ def test_bits_tile_kernel_equals_popcount_kernel(B, n, m, d, kind, code):
     ref = _bits_call(x1, x2, kind, code, True)
     assert torch.equal(torch.nan_to_num(tile, nan=-7.0).view(torch.int32),
                        torch.nan_to_num(ref, nan=-7.0).view(torch.int32))
+
+
+# Ragged output rows of at most 256 features: few rows leave by dwords (the aligned stores' blocks would
+# be nearly empty), more by aligned whole lines; the bits of the same columns among m + 1 (m % 4 == 0).
+@pytest.mark.parametrize("B,n,m,d,lines", [(1, 1, 70003, 166, False), (1, 43, 70003, 166, False), (1, 44, 70003, 166, True),
+                                           (1, 25, 70003, 60, False), (1, 26, 70003, 60, True), (9, 5, 3003, 166, False),
+                                           (1, 5, 3003, 166, True), (1, 300, 20003, 250, True), (3, 257, 3003, 33, True)])
+def test_popcount_ragged_rows(B, n, m, d, lines):
+    x1, x2 = (rand(B, n, d, seed=7) < 0.3).to(DEV), (rand(B, m + 1, d, seed=8) < 0.3).to(DEV)
+    x2m = x2[:, :m].contiguous()
+    want = torch.ops.torchpairwise.hamming_distances(x1, x2)[..., :m]
+    for family, count in (("bool_reduce_kernel", 1), ("bool_reduce_ragged_kernel", int(lines))):
+        with Launches(family) as launches:
+            got = torch.ops.torchpairwise.hamming_distances(x1, x2m)
+        assert launches.count == count
+        assert torch.equal(got, want)
 
 
 # --------------------------------------------------------------------------------------

@@ -363,12 +363,21 @@ int launch_reduce(const uint32_t *a, const uint32_t *b, const int32_t *pa, const
     const double inv_d = d < (int64_t)kFloatExactLimit ? 1.0 / (double)d : 0.0;
     const float inv_df = 1.0f / (float)d;  // as ATen's host-side reciprocal of a CPU scalar
     const bool vec_store = (m % 4 == 0) && aligned16(out);
-    const LaunchEvents ev = launch_events("bool_reduce_kernel");
-    const int64_t grid_y = vec_store ? cdiv(n, 32) : cdiv(n, 256) * 8;
-    if (W <= 8 && m > 256 && grid_y <= kMaxGridYZ) {
+    // RAGGED's blocks hold 8 rows each of 4 of 32 residues, so few rows leave most of a block's rows
+    // empty and eight blocks stage the same columns: it takes 44 rows or more, 26 of one 16-byte
+    // piece, and few columns (blocks for 256 CUs at most).  Else the rows leave in dwords
+    // (hamming, a call, dwords -> RAGGED: n x 1000003 x 166, n = 1 208 -> 374 us, 40 377 -> 386, 48 394
+    // -> 386, 64 461 -> 389; x 60, n = 24 177 -> 189, 32 220 -> 192; 16 x 3001 x 166 18.1 -> 16.5).
+    const int64_t ragged_cols = cdiv(m + 31, 512);
+    const bool ragged = !vec_store && (n >= (W <= 4 ? 26 : 44) || ragged_cols * batch <= 32);
+    const int64_t grid_y = ragged ? cdiv(n, 256) * 8 : cdiv(n, 32);
+    const bool wide_tiles = W <= 8 && m > 256 && grid_y <= kMaxGridYZ;
+    const LaunchEvents ev = launch_events(wide_tiles && ragged ? "bool_reduce_ragged_kernel" : "bool_reduce_kernel",
+                                          "bool_reduce_kernel");
+    if (wide_tiles) {
         // ragged: a row's columns begin up to 31 floats before a tile's
-        dim3 grid((unsigned)cdiv(vec_store ? m : m + 31, 512), (unsigned)grid_y, (unsigned)batch);
-        if (!vec_store)
+        dim3 grid((unsigned)(ragged ? ragged_cols : cdiv(m, 512)), (unsigned)grid_y, (unsigned)batch);
+        if (ragged)
             hipExtLaunchKernelGGL((bool_reduce_kernel<OP, EPI, 64, 2, true>), grid, dim3(kThreads), 0, s, ev.start,
                                   ev.stop, 0, a, b, pa, pb, n, m, W, d, inv_d, inv_df, out, vec_store);
         else
