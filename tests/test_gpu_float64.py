@@ -219,10 +219,14 @@ def test_hausdorff_exact_shuffle_equals_cpu_op(dtype):
 
 @pytest.mark.parametrize("shape,kind", [(((2, 3, 2000, 3), (2, 2, 1500, 3)), "random"),
                                         (((1, 2, 700, 2), (1, 3, 650, 2)), "ties"),
-                                        (((1, 4, 1000, 5), (1, 3, 1200, 5)), "random")])
+                                        (((1, 4, 1000, 5), (1, 3, 1200, 5)), "random"),
+                                        # large enough for the cell grid
+                                        (((1, 2, 6000, 3), (1, 3, 9000, 3)), "random"),
+                                        (((2, 2, 64, 2), (2, 2, 30000, 2)), "ties")])
 def test_hausdorff_exact_f32_equals_pruned_pipeline(shape, kind):
     """Two independent GPU implementations of the same loop: the exact-order wave kernel in
-    float32 and the pruned cell-grid pipeline (the float32 op) agree bit for bit."""
+    float32 and the float32 op (the dense kernels on small clouds, the pruned cell grid on large
+    ones, the generic scan at d = 5) agree bit for bit."""
     g = _g(51)
     s1, s2 = shape
     if kind == "ties":

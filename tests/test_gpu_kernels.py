@@ -425,8 +425,8 @@ def test_hausdorff_clustered_bit_exact(d):
 
 @pytest.mark.parametrize("d", [1, 2, 3])
 def test_hausdorff_self_distance_bit_exact(d):
-    """x2 = x1: every min is 0 and T stays 0, so no m can be dropped: every m goes through the
-    second pass and its full scan, and the tie rules pick the indices."""
+    """x2 = x1 on the dense kernels: every min is 0, and the tie rules pick the indices (on the
+    grid: test_hausdorff_grid_self_bit_exact)."""
     g = torch.Generator().manual_seed(40 + d)
     x = torch.rand(2, 3000, d, generator=g)
     x[:, 100:110] = x[:, 200:210]  # duplicated points
@@ -439,7 +439,8 @@ def test_hausdorff_self_distance_bit_exact(d):
 
 @pytest.mark.parametrize("shape", [
     (None, 2, 700, 2, 900, 4),      # d = 4: parallel seeds and final rescan, plain scan
-    (1100, 1, 40, 1, 50, 2),        # 2200 clouds to sort: one block per cloud
+    (1100, 1, 40, 1, 50, 2),        # 1100 pairs of clouds on the dense kernels
+    (1030, 1, 600, 1, 4096, 2),     # 2060 clouds to sort: one block per cloud
     (None, 64, 65537, 64, 4, 2),    # pairs x p1 > 2^28: x1 unsorted, leftovers in the wave
     (None, 1, 9000, 1, 70000, 3),   # seeds over 3 x1 chunks, rescan over 18 x2 chunks
     (None, 3, 20000, 3, 20000, 3),  # the bench's layout: m with min >= T go to the survivor list
@@ -456,10 +457,9 @@ def test_hausdorff_plan_variants_bit_exact(shape):
 
 @pytest.mark.parametrize("case", ["offset", "flat", "tiny_x2", "one_x2", "shuffled_many_clouds"])
 def test_hausdorff_cell_scan_edges_bit_exact(case):
-    """Cases aimed at the sorted mode's whole-cell test (an x1 cell's exact box against x2
-    points) and its window pass: coordinates far from the origin (rounding of every difference),
-    an axis with zero span (one cell along it), x2 clouds of fewer points than the cell test
-    takes, and a shuffle through the one-block-per-cloud sort."""
+    """Coordinates far from the origin (rounding of every difference), an axis with zero span, x2
+    clouds of three points and of one, and a shuffle over many clouds, all on the dense kernels
+    (on the grid: the test of these names below)."""
     g = torch.Generator().manual_seed(77)
     perm1 = perm2 = None
     if case == "offset":
@@ -490,9 +490,9 @@ def test_hausdorff_cell_scan_edges_bit_exact(case):
 
 
 def _hd_nonfinite(case):
-    """Inputs holding NaN, +-inf, or coordinates whose squared differences overflow, for each
-    launch plan: the sorted mode (d <= 3, few pairs), d = 4 (seeds and scan without the grid),
-    d = 5 (the generic scan) and the unsorted cell scan (pairs x p1 > 2^28)."""
+    """Inputs holding NaN, +-inf, or coordinates whose squared differences overflow, for the dense
+    kernels (small clouds, d <= 3; the sorted grid has a test of its own below), d = 4 (seeds and
+    scan without the grid), d = 5 (the generic scan) and the unsorted cell scan (pairs x p1 > 2^28)."""
     g = torch.Generator().manual_seed(91)
     perm1 = perm2 = None
     x1 = torch.rand(3, 500, 3, generator=g)
@@ -583,19 +583,103 @@ def test_hausdorff_dense_bit_exact(p1, p2, d, case):
         x1[1, 0, p1 // 2, d - 1] = float("nan")
     elif case == "inf_x2":
         x2[0, 2, p2 - 1, 0] = float("inf")
-    _hd_check(x1, x2, perm1, perm2, f"{case} {p1}x{p2}x{d}")
+    _hd_check(x1, x2, perm1, perm2, f"{case} {p1}x{p2}x{d}", grid=False)
 
 
-def _hd_check(x1, x2, perm1, perm2, what):
+def _hd_check(x1, x2, perm1, perm2, what, grid=None):
+    """Against the loop itself; grid: whether the grid is expected to run (its ten or more launches) or
+    the dense kernels (two)."""
     dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
     host = lambda t: None if t is None else t.numpy()  # noqa: E731
+    print(what, tuple(x1.shape), tuple(x2.shape), flush=True)
+    c = capi.HausdorffCounters().arm()
     got = capi.directed_hausdorff(x1.to(DEV), x2.to(DEV), dev(perm1), dev(perm2))
+    launches = c.read()["launches"]
+    assert grid is None or (launches > 2) == grid, launches
     want = cref.directed_hausdorff(x1.numpy(), x2.numpy(), host(perm1), host(perm2), threads=8)
     for g, w, nm in zip(got, want, ("value", "idx1", "idx2")):
         assert_equal(g.cpu(), torch.from_numpy(w), f"{what} {nm}", nan_payload=False)
 
 
-# the grid's sorted mode at one pair of clouds past the dense kernels' 2^28 point pairs
+@pytest.mark.parametrize("d", [1, 2, 3])
+def test_hausdorff_grid_self_bit_exact(d):
+    """x2 = x1 on the sorted grid: every min is 0 and T stays 0, so no m can be dropped: every m goes
+    through the second pass and its full scan, and the tie rules pick the indices."""
+    x = rand(2, 9000, d, seed=40 + d)
+    x[:, 100:110] = x[:, 200:210]  # duplicated points
+    _hd_check(x, x.clone(), None, None, f"self d={d}", grid=True)
+
+
+# Few x1 points against a long x2 (the dense kernels' blocks would be too few), so that the loop that
+# follows the reference's order stays short where a value is not finite
+@pytest.mark.parametrize("case", ["nan_x1", "nan_x2", "nan_x2_last", "inf_x1", "ninf_x2", "nan_cloud", "overflow",
+                                  "overflow_rows", "mixed_d1", "mixed_d2", "batched", "shuffled"])
+def test_hausdorff_grid_nonfinite_bit_exact(case):
+    """NaN, infinities and overflow on the sorted grid (see test_hausdorff_nonfinite_bit_exact)."""
+    nan, inf = float("nan"), float("inf")
+    perm1 = perm2 = None
+    x1, x2 = _hd_inputs(None, 3, 64, 2, 20000, 3, seed=91)
+    if case == "nan_x1":
+        x1[0, 10, 1] = nan
+    elif case == "nan_x2":
+        x2[1, 7, 0] = nan
+    elif case == "nan_x2_last":
+        x2[0, -1, 2] = nan
+    elif case == "inf_x1":
+        x1[1, 33, 0] = inf
+    elif case == "ninf_x2":
+        x2[0, 5, 1] = -inf
+    elif case == "nan_cloud":
+        x1[2] = nan
+    elif case == "overflow":
+        x1, x2 = x1 * 1e20, x2 * -1e20
+    elif case == "overflow_rows":
+        x1[0, 40:43] = 3e38
+    elif case == "mixed_d1":
+        x1, x2 = _hd_inputs(None, 2, 33000, 2, 60, 1, seed=92)
+        x1[0, 3, 0] = nan
+        x2[1, 9, 0] = inf
+    elif case == "mixed_d2":
+        x1, x2 = _hd_inputs(None, 2, 64, 2, 30000, 2, seed=92)
+        x1[0, 3, 0] = nan
+        x2[1, 9, 0] = inf
+    elif case == "batched":  # only batch 1 holds a NaN: batches 0 and 2 keep the pruned path
+        x1, x2 = _hd_inputs(3, 2, 64, 2, 20000, 3, seed=93)
+        x1[1, 0, 17, 2] = nan
+    else:
+        x1, x2 = _hd_inputs(2, 2, 64, 3, 20000, 3, seed=94)
+        x2[0, 1, 50, 0] = nan
+        x1[1, 1, 60, 1] = -inf
+        perm1, perm2 = P.hausdorff_permutations(2, 64, 20000, torch.Generator().manual_seed(6))
+    _hd_check(x1, x2, perm1, perm2, case, grid=True)
+
+
+@pytest.mark.parametrize("case", ["offset", "flat", "tiny_x2", "one_x2", "clouds", "shuffled_many_clouds"])
+def test_hausdorff_grid_cell_scan_edges_bit_exact(case):
+    """Cases aimed at the sorted mode's whole-cell test (an x1 cell's exact box against x2 points) and
+    its window pass: coordinates far from the origin, an axis with zero span (one cell along it), x2
+    clouds of fewer points than the cell test takes, several shuffled clouds, and a shuffle through
+    the one-block-per-cloud sort."""
+    perm1 = perm2 = None
+    if case in ("offset", "flat", "clouds"):
+        x1, x2 = _hd_inputs(2, 2, 6000, 3, 9000, 3, seed=77)
+        if case == "offset":
+            x1, x2 = x1 + 1.0e4, x2 + 1.0e4
+        elif case == "flat":
+            x1[..., 2] = x2[..., 2] = 0.25
+        else:
+            perm1, perm2 = P.hausdorff_permutations(2, 6000, 9000, torch.Generator().manual_seed(8))
+    elif case == "tiny_x2":
+        x1, x2 = _hd_inputs(None, 2, 33000, 3, 3, 3, seed=78)
+    elif case == "one_x2":
+        x1, x2 = _hd_inputs(None, 2, 33000, 2, 1, 2, seed=79)
+    else:
+        x1, x2 = _hd_inputs(1030, 1, 600, 1, 4096, 3, seed=80)
+        perm1, perm2 = P.hausdorff_permutations(1030, 600, 4096, torch.Generator().manual_seed(8))
+    _hd_check(x1, x2, perm1, perm2, case, grid=True)
+
+
+# the sorted grid at one pair of clouds past the dense kernels' 2^28 point pairs
 @pytest.mark.parametrize("case", ["offset", "flat", "shuffled", "ties", "self", "nan_x1"])
 def test_hausdorff_grid_above_dense_bit_exact(case):
     x1, x2 = _hd_inputs(None, 1, 17000, 1, 16500, 3, seed=60)
@@ -613,7 +697,7 @@ def test_hausdorff_grid_above_dense_bit_exact(case):
     else:
         x1[0, 5, 1] = float("nan")
         x1[0, 6:] = x1[0, 6:] * 0.1  # short early exits: the loop itself runs on one wave
-    _hd_check(x1, x2, perm1, perm2, case)
+    _hd_check(x1, x2, perm1, perm2, case, grid=True)
 
 
 # Which calls evaluate every point pair (two launches): those that cost less so than the grid's

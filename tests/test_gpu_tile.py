@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+
 class Launches:
     """The launches of one kernel family inside a ``with`` block: which path a call took."""
 
@@ -65,21 +66,24 @@ def _same_bits(a, b):
     return torch.equal(ia, ib)
 
 
+# batches of more than 256 tiles of 128 x 128, which the small-output kernel does not take
 @pytest.mark.parametrize("dtype,B,n,m,d", [
-    (torch.float32, 1, 300, 260, 32),
-    (torch.float32, 2, 129, 136, 96),
-    (torch.float32, 1, 128, 256, 256),
-    (torch.float32, 1, 130, 260, 512),     # 16 chunks: the double-buffered long-K variant
-    (torch.bfloat16, 1, 300, 264, 64),
-    (torch.bfloat16, 3, 257, 520, 192),
-    (torch.bfloat16, 1, 128, 128, 256),
-    (torch.bfloat16, 1, 200, 136, 1024),   # long K
-    # bf16 ragged rows (m % 8 = 1 .. 7): whole units funnel-shifted, head / tail values
-    (torch.bfloat16, 1, 300, 259, 64),
-    (torch.bfloat16, 2, 129, 133, 192),
-    (torch.bfloat16, 1, 130, 262, 1024),
-    (torch.bfloat16, 1, 70, 7, 128),
-    (torch.bfloat16, 1, 257, 140, 256),
+    (torch.float32, 29, 300, 260, 32),
+    (torch.float32, 65, 129, 136, 96),
+    (torch.float32, 129, 128, 256, 256),
+    (torch.float32, 43, 130, 260, 512),     # 16 chunks: the double-buffered long-K variant
+    (torch.float32, 29, 300, 259, 64),      # ragged rows: 16-byte units at any dword
+    (torch.float32, 65, 129, 142, 512),
+    (torch.bfloat16, 29, 300, 264, 64),
+    (torch.bfloat16, 18, 257, 520, 192),
+    (torch.bfloat16, 257, 128, 128, 256),
+    (torch.bfloat16, 65, 200, 136, 1024),   # long K
+    # bf16 ragged rows (m % 8 = 1 .. 7): 16-byte units at any value
+    (torch.bfloat16, 29, 300, 259, 64),
+    (torch.bfloat16, 65, 129, 133, 192),
+    (torch.bfloat16, 43, 130, 262, 1024),
+    (torch.bfloat16, 257, 70, 7, 128),
+    (torch.bfloat16, 43, 257, 140, 256),
 ])
 @pytest.mark.parametrize("epi", EPIS)
 def test_inner_tile_kernel_equals_staged_kernel(dtype, B, n, m, d, epi):
@@ -88,9 +92,19 @@ def test_inner_tile_kernel_equals_staged_kernel(dtype, B, n, m, d, epi):
     x2[:, 3] = 0  # a zero row: the guarded cosine divide
     if m > 7:
         x2[:, 7] = x1[:, 0]  # an identical pair: the clamped euclidean floor
-    tile = _inner(x1, x2, epi, False)
-    staged = _inner(x1, x2, epi, True)
-    assert _same_bits(tile, staged)
+    with Launches("inner_tile_kernel") as on_tile:
+        tile = _inner(x1, x2, epi, False)
+    with Launches("pairwise_inner_kernel") as on_staged:
+        staged = _inner(x1, x2, epi, True)
+    with Launches("inner_small_kernel") as on_small:
+        _inner(x1, x2, epi, False), _inner(x1, x2, epi, True)
+    assert (on_tile.count, on_staged.count, on_small.count) == (1, 1, 0)
+    if dtype == torch.bfloat16 and epi >= capi.EPI_COSINE_SIM:
+        # tiles without a zero row divide by reciprocal norms (2 ulp of float, 2^-22 near 1, before the
+        # bf16 rounding): one bf16 ulp, 2^-7 relative, or 2^-21 where 1 - q cancels
+        assert torch.allclose(tile.float(), staged.float(), rtol=2.0 ** -7, atol=2.0 ** -21)
+    else:
+        assert _same_bits(tile, staged)
 
 
 # Small outputs (64 x 64 tiles, norms formed in the kernel or given) against the 128 x 128 kernels,
@@ -188,7 +202,7 @@ BITS_CASES = ([("metric", k) for k in range(10)] + [("jaccard", 0)] +
 @pytest.mark.parametrize("B,n,m,d", [(1, 130, 132, 1), (1, 70, 136, 33), (2, 129, 136, 128), (1, 130, 132, 256),
                                      (1, 300, 260, 257), (2, 129, 136, 1024), (1, 130, 132, 1500),
                                      (1, 70, 132, 2081),
-                                     # ragged rows (m % 4 != 0): dword row stores
+                                     # ragged rows (m % 4 != 0): dword rows (counts) or unaligned units
                                      (1, 130, 131, 1024), (2, 70, 133, 300), (1, 129, 130, 100),
                                      (1, 257, 259, 33), (1, 40, 1, 512)])
 @pytest.mark.parametrize("kind,code", BITS_CASES)
@@ -220,12 +234,11 @@ def test_popcount_ragged_rows(B, n, m, d, lines):
 
 
 # --------------------------------------------------------------------------------------
-# fp32 backward on the matrix-core tile kernels: the weights formed inside the grad_x1 product
-# (euclidean, sqeuclidean, polynomial, sigmoid; 128 x 256 tiles, two column tiles at d = 300),
-# x2 (for grad_x1) and W, x1 (for grad_x2) read k-major in place; inputs offset by one element
-# take the weight pass and the split-K GEMM instead.
+# fp32 backward of small problems with aligned inputs and with inputs offset by one element: the
+# weight pass and the split-K GEMM (polynomial), op_backward_kernel with whole and element loads
+# (the others; the kernels of larger problems are in test_backward_paths_of_large_problems).
 # Bar: float64 autograd of the reference's composite on the CPU, rtol 1e-4 (+ 1e-4 * max);
-# the two device paths agree to 1e-5 * max (different summation orders).
+# the two calls agree to 1e-5 * max (different summation orders).
 # --------------------------------------------------------------------------------------
 BWD_OPS = [("euclidean_distances", {}), ("sqeuclidean_distances", {}), ("cosine_distances", {}),
            ("cosine_similarity", {}), ("correlation_distances", {}),
@@ -262,9 +275,9 @@ def test_backward_products_tile_fp32(name, kw, B, n, m, d):
     for k, want in enumerate((ra.grad, rb.grad)):
         tile, split = grads[False][k], grads[True][k]
         scale = float(want.abs().max())
-        assert_close(tile, want, rtol=1e-4, atol=1e-4 * scale, what=f"{name} grad_x{k + 1} (tile)")
-        assert_close(split, want, rtol=1e-4, atol=1e-4 * scale, what=f"{name} grad_x{k + 1} (split-K)")
-        assert_close(tile, split.double(), rtol=0, atol=1e-5 * scale, what=f"{name} grad_x{k + 1} tile vs split-K")
+        assert_close(tile, want, rtol=1e-4, atol=1e-4 * scale, what=f"{name} grad_x{k + 1} (aligned)")
+        assert_close(split, want, rtol=1e-4, atol=1e-4 * scale, what=f"{name} grad_x{k + 1} (offset)")
+        assert_close(tile, split.double(), rtol=0, atol=1e-5 * scale, what=f"{name} grad_x{k + 1} aligned vs offset")
 
 
 # Both gradients in one launch (op_backward_kernel): edges of its 64-row tiles, 64- and 128-feature
@@ -346,14 +359,77 @@ def test_backward_passes_above_one_launch(name, dtype, n, m, d):
         assert_close(got.float(), want, rtol=tol, atol=tol * float(want.abs().max()), what=name)
 
 
-# bf16: x2 (for grad_x1) and W, x1 (for grad_x2) read k-major through transposing LDS reads,
-# and (euclidean, sigmoid; n % 128 == 0) the weights formed inside the grad_x1 product, against
-# the path that inputs offset by one element take (W^T and transposed copies of x1, x2
-# written first, and the register-staged kernel for their misaligned X); bar: the bf16 tolerance
-# against float64 autograd, 1e-2 (+ 1e-2 * max), and the two device paths within one bf16 ulp of
-# each other (2^-7 relative, the ulp of values in [1, 2), + 1e-3 * max).  (1, 128, 65536, 256):
-# grad_x2's product (M = 65536, N = 256, K = 128) has 512 tiles of 128 x 256, enough to fill the
-# GPU, and takes the 128 x 256 bf16 product kernel
+# The backward's kernels for problems past op_backward_kernel's limit, each with aligned inputs and
+# with inputs offset by one element, which take the weight pass and the split-K GEMM (fp32) or W^T,
+# transposed copies and the register-staged kernel (bf16):
+#   fused:  the weights formed inside the grad_x1 product (128 x 256 tiles that fill the GPU), grad_x2
+#           on the 128 x 128 tile kernel, W and x1 read k-major in place;
+#   tiles:  half as many 128 x 256 tiles, so the weight pass, then both products on the tile kernel;
+#   wide:   bf16's fused path with grad_x2 on 128 x 256 tiles;
+#   passes: ragged sizes in two batches, where both inputs take the offset inputs' path.
+# The tile kernels' launches in the backward tell the paths apart.  Bar: float64 autograd of plain
+# torch on the GPU, rtol 1e-4 or 1e-2 (+ that times the largest).
+PATHS = {"fused": (2, 4096, 2048, 2048), "tiles": (1, 4096, 4096, 2048), "wide": (1, 8192, 8192, 2048),
+         "passes": (2, 3101, 3003, 300)}
+
+
+def _op64(name, kw, a, b):
+    """The named metric of one batch in plain torch (float64 inputs)."""
+    if name == "correlation_distances":
+        a, b = a - a.mean(1, keepdim=True), b - b.mean(1, keepdim=True)
+    s = a @ b.T
+    if "euclidean" in name:
+        sq = (a.square().sum(1)[:, None] + b.square().sum(1)[None] - 2 * s).clamp_min(0)
+        return sq if name.startswith("sq") else sq.sqrt()
+    if name.startswith(("cosine", "correlation")):
+        s = s / (a.norm(dim=1)[:, None] * b.norm(dim=1)[None])
+        return s if name == "cosine_similarity" else 1 - s
+    if name == "linear_kernel":
+        return s
+    return (s * kw["gamma"] + 1).pow(kw["degree"]) if name == "polynomial_kernel" else (s * kw["gamma"] + 1).tanh()
+
+
+@pytest.mark.parametrize("path,dtype", [(p, t) for p in PATHS for t in (torch.float32, torch.bfloat16)
+                                        if p != "wide" or t == torch.bfloat16])
+@pytest.mark.parametrize("name,kw", BWD_OPS)
+def test_backward_paths_of_large_problems(name, kw, path, dtype):
+    import torchpairwise_amd as tp
+    from tests._util import assert_close
+
+    B, n, m, d = PATHS[path]
+    print(f"{path} {name} {dtype} B={B} n={n} m={m} d={d}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(5)
+    x1, x2, g = (torch.randn(B, r, c, generator=gen, device=DEV).to(dtype) for r, c in ((n, d), (m, d), (n, m)))
+    want = ([], [])
+    for i in range(B):
+        ra, rb = x1[i].double().requires_grad_(), x2[i].double().requires_grad_()
+        for lst, t in zip(want, torch.autograd.grad(_op64(name, kw, ra, rb), (ra, rb), g[i].double())):
+            lst.append(t)
+    tol = 1e-4 if dtype == torch.float32 else 1e-2
+    for offset in (False, True):
+        a, b = _leaf(x1, offset), _leaf(x2, offset)
+        out = getattr(tp, name)(a, b, **kw)
+        count = {}
+        for family in ("op_backward_kernel", "inner_tile_kernel", "grad_wide_bf16_kernel"):
+            with Launches(family) as launches:
+                got = torch.autograd.grad(out, (a, b), g, retain_graph=True)
+            count[family] = launches.count
+        print(offset, count, flush=True)
+        assert count["op_backward_kernel"] == 0
+        # (sqeuclidean takes the power-sum kernels, polynomial and linear other mixes of these products)
+        if name.startswith(("euclidean", "cosine", "correlation", "sigmoid")) and not offset:
+            tiles, wide = {"fused": (1, 0), "tiles": (2, 0), "wide": (0, 1), "passes": (0, 0)}[path]
+            assert (count["inner_tile_kernel"], count["grad_wide_bf16_kernel"]) == (tiles, wide)
+        for k in (0, 1):
+            w = torch.stack(want[k])
+            assert_close(got[k].float(), w, rtol=tol, atol=tol * float(w.abs().max()),
+                         what=f"{name} {path} offset={offset} grad_x{k + 1}")
+
+
+# bf16 backward of small problems with aligned inputs and with inputs offset by one element
+# (polynomial: the weight pass and the products; the others: op_backward_kernel with whole and element
+# loads): bar: the bf16 tolerance against float64 autograd, 1e-2 (+ 1e-2 * max), and the two calls
+# within one bf16 ulp of each other (2^-7 relative, the ulp of values in [1, 2), + 1e-3 * max).
 @pytest.mark.parametrize("B,n,m,d", [(2, 128, 192, 64), (1, 1088, 1024, 72), (1, 256, 128, 264), (1, 128, 65536, 256)])
 @pytest.mark.parametrize("name", ["euclidean_distances", "cosine_distances", "polynomial_kernel", "sigmoid_kernel"])
 def test_backward_products_kmajor_bf16(name, B, n, m, d):
@@ -376,19 +452,20 @@ def test_backward_products_kmajor_bf16(name, B, n, m, d):
     for k, want in enumerate((ra.grad, rb.grad)):
         kmaj, other = grads[False][k], grads[True][k]
         scale = float(want.abs().max())
-        assert_close(kmaj, want, rtol=1e-2, atol=1e-2 * scale, what=f"{name} grad_x{k + 1} (k-major)")
+        assert_close(kmaj, want, rtol=1e-2, atol=1e-2 * scale, what=f"{name} grad_x{k + 1} (aligned)")
         assert_close(kmaj, other.double(), rtol=2.0 ** -7, atol=1e-3 * scale,
-                     what=f"{name} grad_x{k + 1} k-major vs transposed")
+                     what=f"{name} grad_x{k + 1} aligned vs offset")
 
 
 # --------------------------------------------------------------------------------------
-# Rows that are not whole 128-byte chunks: for outputs of 2^20 entries or more the public
-# inner-product ops copy the operands zero-padded to whole chunks and take the tile kernel;
-# below that, the staged kernel, which zero-fills its last chunk.  Bit-identical either way.
+# Rows that are not whole 128-byte chunks: for outputs of 2^20 entries or more that the
+# small-output kernel does not take, the public inner-product ops copy the operands zero-padded to
+# whole chunks and take the tile kernel, against the staged kernel of the C entry, which zero-fills
+# its last chunk.  Bit-identical either way.
 # --------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype,n,m,d", [
-    (torch.float32, 1100, 1000, 127), (torch.float32, 1024, 1040, 130), (torch.float32, 1030, 1024, 1),
-    (torch.bfloat16, 1030, 1024, 255), (torch.bfloat16, 1024, 1032, 200),
+    (torch.float32, 2100, 2000, 127), (torch.float32, 2049, 2080, 130), (torch.float32, 2060, 2048, 1),
+    (torch.float32, 2050, 2047, 700), (torch.bfloat16, 2060, 2048, 255), (torch.bfloat16, 2049, 2056, 200),
 ])
 @pytest.mark.parametrize("op,epi", [("euclidean_distances", capi.EPI_EUCLIDEAN),
                                     ("cosine_similarity", capi.EPI_COSINE_SIM),
@@ -398,6 +475,12 @@ def test_padded_rows_equal_staged_kernel(dtype, n, m, d, op, epi):
     x1 = randn(1, n, d, seed=11).to(DEV, dtype)
     x2 = randn(1, m, d, seed=12).to(DEV, dtype)
     x2[:, 5] = x1[:, 0]
-    got = getattr(torch.ops.torchpairwise, op)(x1[0], x2[0])
-    assert _same_bits(got, _inner(x1, x2, epi, True)[0])
+    with Launches("inner_tile_kernel") as on_tile:
+        got = getattr(torch.ops.torchpairwise, op)(x1[0], x2[0])
+    with Launches("inner_small_kernel") as on_small:
+        getattr(torch.ops.torchpairwise, op)(x1[0], x2[0])
+    with Launches("pairwise_inner_kernel") as on_staged:
+        want = _inner(x1, x2, epi, True)[0]
+    assert (on_tile.count, on_small.count, on_staged.count) == (1, 0, 1)
+    assert _same_bits(got, want)
 
