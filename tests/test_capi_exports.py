@@ -47,6 +47,16 @@ def test_hausdorff_workspace_fits_the_static_buffer():
         assert l.tpw_hausdorff_workspace_size(*sizes) <= 96 << 20, sizes
 
 
+def test_lp_backward_splits_fill_three_blocks():
+    """The Lp backward's workspace holds the narrow kernel's partials for three blocks per CU (256 CUs):
+    8 splits of 12000 x 12000 x 64 (94 row blocks), 6 of 16384^2 x 16, 12 of 8192^2 x 64 (regression: it
+    was split for two, up to 11 % slower)."""
+    l = _capi.lib()
+    for n, d, splits in ((12000, 64, 8), (16384, 16, 6), (8192, 64, 12)):
+        size = l.tpw_lp_backward_workspace_size(1, n, n, d) - 4 * n * n  # beside the weights
+        assert splits * 4 * n * d <= size < (splits + 1) * 4 * n * d
+
+
 def test_small_output_rule():
     """Where the 64 x 64 inner-product kernel runs (256 CUs): not where the 128 x 128 tile kernel,
     padded copies or not, takes less (regression: wide rows went there, up to 2.2 times as slow)."""

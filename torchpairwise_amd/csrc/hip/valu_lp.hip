@@ -24,6 +24,7 @@
 // p = 2, 3 and general p > 2 (and p = 1 where its range scan allows) own 128 features a block.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -637,8 +638,12 @@ __global__ void pair_weight_kernel(const float *__restrict__ g, const float *__r
 // earlier launch choosing which one computes).
 // WHOLE: n, m and d are multiples of 4 (and the staging offsets 32-bit), so each 16-byte staging
 // load lies whole in its array or whole past its end, where it reads 0, and needs no test.
+// Three waves per SIMD for the narrow instances (168 VGPRs, two more spilled by canberra's and p = 1's),
+// two for the wide ones and for the p = 1 fallback with the exp-scaled gradient.
+template <int PK, int FW, bool EXPG>
+constexpr int kBwdWaves = (FW == kBFeatWide || (EXPG && PK == kP1)) ? 2 : 3;
 template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW = kBFeat, bool EXPG = false, bool WHOLE = false>
-__global__ __launch_bounds__(kThreads, 2) void lp_backward_kernel(
+__global__ __launch_bounds__(kThreads, (kBwdWaves<PK, FW, EXPG>)) void lp_backward_kernel(
     const float *__restrict__ g, const float *__restrict__ aux0, const float *__restrict__ aux1,
     const float *__restrict__ x1, const float *__restrict__ x2, const float *__restrict__ w,
     int64_t n, int64_t m, int64_t d, float p, int64_t j_per_split, int64_t batch,
@@ -1123,12 +1128,6 @@ int fill(float *p, int64_t len, float v, hipStream_t s) {
     return check_launch("fill_kernel");
 }
 
-// Blocks of the backward grid per CU that the split count aims at: two, which every instance
-// fits at once.  A constant and not each instance's occupancy, so that two instances of one
-// backward (the exp-scaled gradient and the plain one) split and so round alike.
-constexpr int kSplitBlocksPerCU = 2;
-
-
 // Number of j splits for `slots` resident blocks: the (row block, feature block, batch)
 // grid alone fills base blocks; splitting j multiplies that, and a whole number of
 // resident rounds avoids a partly filled last round.  A split is a whole number of kBJ-pair
@@ -1137,7 +1136,7 @@ constexpr int kSplitBlocksPerCU = 2;
 // blocks (32 or 64 KB each) take a few us to add (manhattan forward and backward 3001 x 1999 x
 // 100: 368 -> 200 us against splits of at least 512 pairs; 3176 x 3178 x 10: 328 -> 120).
 constexpr int64_t kMaxSplits = 64;
-int64_t lp_backward_splits(int64_t slots, int64_t batch, int64_t n, int64_t m, int64_t d, int64_t fw) {
+int64_t splits_for_slots(int64_t slots, int64_t batch, int64_t n, int64_t m, int64_t d, int64_t fw) {
     const int64_t base = cdiv(n, kBRows) * cdiv(d, fw) * batch;
     if (base == 0 || m == 0) return 1;  // nothing to split
     int64_t splits = base >= slots ? 1 : slots / base;
@@ -1148,7 +1147,23 @@ int64_t lp_backward_splits(int64_t slots, int64_t batch, int64_t n, int64_t m, i
     const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
     return cdiv(m, jps);
 }
-int64_t split_slots() { return (int64_t)device_cus() * kSplitBlocksPerCU; }
+// Two blocks per CU are resident of every instance, three of the narrow kernel's; a stage of three
+// takes `third` times as long as one of two (1.31 p = 1.5 to 1.5 canberra, measured at 8192^2 to 16384^2),
+// so as many splits as fill three are taken where their fewer stages make up for that.  Backward,
+// two -> three: p = 1.5 8192^2 x 64 4869 -> 4366 us, chebyshev 12000 x 11999 x 128 8899 -> 6367, braycurtis
+// 15744 -> 11499; canberra 9000 x 9001 x 30 stays at two (10760 against 11360).  From the sizes and the
+// metric alone, so that two instances of one backward (the exp-scaled gradient and the plain one)
+// split and so round alike.
+int64_t lp_backward_splits(double third, int64_t batch, int64_t n, int64_t m, int64_t d, int64_t fw) {
+    const int64_t cus = device_cus();
+    const int64_t two = splits_for_slots(2 * cus, batch, n, m, d, fw);
+    if (fw == kBFeatWide) return two;
+    const int64_t three = splits_for_slots(3 * cus, batch, n, m, d, fw);
+    auto stages = [m](int64_t splits) { return (double)cdiv(cdiv(m, splits), kBJ); };
+    return third * stages(three) < stages(two) ? three : two;
+}
+template <int MODE, int PK>
+constexpr double kThird = MODE == kCanberra || PK == kP1 || PK == kP3 ? 1.48 : 1.4;
 
 // grad [batch, n, d] of the first operand (x2's gradient: pass x2 as x1, n <-> m, TR).
 template <int MODE, int PK, bool TR, bool WGRAD, bool PRE, int FW, bool EXPG = false, bool WHOLE = false>
@@ -1164,7 +1179,7 @@ int launch_backward(const float *g, const float *aux0, const float *aux1, const 
     // layout and the one sum_splits pass after the last)
     int64_t splits = shared_splits && *shared_splits > 0
                          ? *shared_splits
-                         : lp_backward_splits(split_slots(), batch, n, m, d, FW);
+                         : lp_backward_splits(kThird<MODE, PK>, batch, n, m, d, FW);
     if (shared_splits) *shared_splits = splits;
     const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
     dim3 grid((unsigned)cdiv(d, FW), (unsigned)cdiv(n, kBRows), (unsigned)(splits * batch));
@@ -1329,14 +1344,14 @@ struct Workspace {
 };
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 Workspace workspace_layout(int metric, int64_t batch, int64_t n, int64_t m, int64_t d) {
-    const int64_t slots = split_slots();
-    // the wide kernel's grid has fewer feature blocks, so it may take more splits
-    int64_t s1 = lp_backward_splits(slots, batch, n, m, d, kBFeatWide);
-    int64_t s2 = lp_backward_splits(slots, batch, m, n, d, kBFeatWide);
-    const int64_t s1n = lp_backward_splits(slots, batch, n, m, d, kBFeat);
-    const int64_t s2n = lp_backward_splits(slots, batch, m, n, d, kBFeat);
-    s1 = s1 > s1n ? s1 : s1n;
-    s2 = s2 > s2n ? s2 : s2n;
+    // the wide kernel's grid has fewer feature blocks, so it may take more splits; the narrow one's
+    // splits are at most those of three blocks per CU
+    const int64_t cus = device_cus();
+    auto most = [&](int64_t rows, int64_t cols) {
+        return std::max(splits_for_slots(2 * cus, batch, rows, cols, d, kBFeatWide),
+                        splits_for_slots(3 * cus, batch, rows, cols, d, kBFeat));
+    };
+    const int64_t s1 = most(n, m), s2 = most(m, n);
     Workspace w{};
     const int64_t part1 = s1 > 1 ? s1 * batch * n * d : 0, part2 = s2 > 1 ? s2 * batch * m * d : 0;
     w.part = align256(sizeof(float) * (size_t)(part1 > part2 ? part1 : part2));
