@@ -61,7 +61,8 @@ int tpw_runtime_version(void);
  * reads the device duration of the launches inside its own timed loop.  Creates events the
  * first time (no device memory).  Not for concurrent use from several threads.
  * Families: "inner_tile_kernel" (the small-output kernel's launches too), "inner_small_kernel"
- * (those alone), "pairwise_inner_kernel", "lp_forward_kernel", "bool_reduce_kernel",
+ * (those alone), "pairwise_inner_kernel", "lp_forward_kernel", "lp_backward_kernel"
+ * ("lp_backward_wide_kernel" and "lp_backward_narrow_kernel"), "bool_reduce_kernel",
  * "bool_reduce_ragged_kernel" (of those, the ragged rows stored in aligned lines),
  * "bool_bits_tile_kernel", "op_backward_kernel", "grad_wide_bf16_kernel". */
 int tpw_launch_timer_arm(const char *family, int capacity);

@@ -218,6 +218,18 @@ def test_lp_backward(p, B, n, m, d, entry):
                      what=f"lp p={p} {nm}")
 
 
+@pytest.mark.parametrize("p,d,wide", [(2.0, 70, 2), (3.0, 65, 2), (2.5, 70, 0), (4.5, 128, 0), (1.5, 128, 0),
+                                      (float("inf"), 70, 0), (3.0, 64, 0)])
+def test_lp_backward_kernel_widths(p, d, wide):
+    """Which p take the 128-feature kernel above 64 features (both directions, no other launch)."""
+    x1, x2, g = (t.to(DEV) for t in (randn(90, d, seed=1), randn(101, d, seed=2), randn(90, 101, seed=3)))
+    dist = capi.lp_distances(x1, x2, p)
+    for family, count in (("lp_backward_wide_kernel", wide), ("lp_backward_narrow_kernel", 2 - wide)):
+        timer = capi.LaunchTimer(family, 8).arm()
+        capi.lp_distances_backward2(g, x1, x2, dist, p)
+        assert len(timer.read()[0]) == count, family
+
+
 def _sign_counts(a, b):
     """sum_j sign(a[i, k] - b[j, k]) with sign(NaN) = 0: the p = 1 gradient for grad = 1."""
     diff = a[:, None, :].astype(np.float64) - b[None, :, :].astype(np.float64)

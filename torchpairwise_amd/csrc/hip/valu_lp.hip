@@ -21,7 +21,7 @@
 // split over several blocks when the row/feature grid alone would not fill the GPU; the
 // per-split partial sums are then added in split order by a second kernel, so the result
 // is deterministic (the reference accumulates with atomics on its GPU path).  Above 64 features
-// p = 2, 3 and general p > 2 (and p = 1 where its range scan allows) own 128 features a block.
+// p = 2 and 3 (and p = 1 where its range scan allows) own 128 features a block.
 #include <math.h>
 
 #include <algorithm>
@@ -581,12 +581,14 @@ __device__ __forceinline__ float fam_term(float a, float b, float w1, float w2, 
 template <int MODE, int PK>
 constexpr bool kPrecomputed = (MODE == kRoot && (PK == kP2 || PK == kP3 || PK == kPLt2 || PK == kPGen)) ||
                               (MODE == kWeighted && PK != kP1) || MODE == kBrayDen;
-// The cases the wide kernel serves (above 64 features): the cdist backward at p = 2, 3 and
-// p > 2 in general, and the p = 2 power sum (sqeuclidean, rbf_kernel).  p = inf (a second
-// per-pair array) and 0 < p < 2 would spill its registers at this width; p = 1 takes it only
-// through run_backward_p1_gated (the sign path alone, chosen by a range scan).
+// The cases the wide kernel serves (above 64 features): the cdist backward at p = 2 and 3, and the
+// p = 2 power sum (sqeuclidean, rbf_kernel).  p = inf (a second per-pair array) and 0 < p < 2 would
+// spill its registers at this width; other p > 2 cost an exponential and a logarithm each, whose
+// chain the narrow kernel's third wave hides better (p = 2.5, wide -> narrow: 8192^2 x 128 6.22 -> 5.66
+// ms, 9000 x 9001 x 70 8.00 -> 7.43); p = 1 takes it only through run_backward_p1_gated (the sign path
+// alone, chosen by a range scan).
 template <int MODE, int PK>
-constexpr bool kWide = (MODE == kRoot && (PK == kP2 || PK == kP3 || PK == kPGen)) || (MODE == kSum && PK == kP2);
+constexpr bool kWide = (MODE == kRoot && (PK == kP2 || PK == kP3)) || (MODE == kSum && PK == kP2);
 
 // VEC: every pointer is 16-byte aligned; four pairs per step with 16-byte accesses, and the
 // len % 4 tail by the first threads.
@@ -1184,8 +1186,10 @@ int launch_backward(const float *g, const float *aux0, const float *aux1, const 
     const int64_t jps = cdiv(cdiv(m, splits), kBJ) * kBJ;
     dim3 grid((unsigned)cdiv(d, FW), (unsigned)cdiv(n, kBRows), (unsigned)(splits * batch));
     float *dst = splits > 1 ? part : grad;
-    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s, g, aux0, aux1, x1, x2, w, n, m, d, (float)p,
-                       jps, batch, dst, eo, es, gate, gate_run);
+    const LaunchEvents ev =
+        launch_events(FW == kBFeatWide ? "lp_backward_wide_kernel" : "lp_backward_narrow_kernel", "lp_backward_kernel");
+    hipExtLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s, ev.start, ev.stop, 0, g, aux0, aux1, x1, x2, w, n, m, d,
+                          (float)p, jps, batch, dst, eo, es, gate, gate_run);
     int rc = check_launch("lp_backward_kernel");
     if (rc != TPW_OK || splits == 1 || !finish) return rc;
     const int64_t len = batch * n * d;
