@@ -322,6 +322,25 @@ def test_lp_backward_p1_wide_gated(entry, outside):
     assert_equal(gx2.cpu(), torch.from_numpy(_sign_counts(b, a).astype(np.float32)), "p=1 grad_x2")
 
 
+@pytest.mark.parametrize("B,n,m,d,launches", [(1, 64, 64, 101, 2), (1, 32, 1, 65, 2), (3, 64, 63, 128, 2),
+                                              (1, 128, 65, 101, 2), (2, 129, 64, 96, 4), (1, 5, 130, 67, 4),
+                                              (1, 200, 64, 64, 2)])
+def test_lp_backward_p1_launches(B, n, m, d, launches):
+    """p = 1 above 64 features: problems of one row block each way take the narrow kernel's two launches
+    alone, larger ones the wide and the narrow kernel behind the range scan.  grad = 1: sign counts bit for bit."""
+    rng = np.random.default_rng(13)
+    a = (rng.integers(-8, 9, size=(B, n, d)) * 0.125).astype(np.float32)
+    b = (rng.integers(-8, 9, size=(B, m, d)) * 0.125).astype(np.float32)
+    x1, x2, g = torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), torch.ones(B, n, m, device=DEV)
+    dist = capi.lp_distances(x1, x2, 1.0)
+    timer = capi.LaunchTimer("lp_backward_kernel", 8).arm()
+    gx1, gx2 = capi.lp_distances_backward2(g, x1, x2, dist, 1.0)
+    assert len(timer.read()[0]) == launches
+    for i in range(B):
+        assert_equal(gx1[i].cpu(), torch.from_numpy(_sign_counts(a[i], b[i]).astype(np.float32)), "grad_x1")
+        assert_equal(gx2[i].cpu(), torch.from_numpy(_sign_counts(b[i], a[i]).astype(np.float32)), "grad_x2")
+
+
 # --------------------------------------------------------------------------------------
 # inner-product backward
 # --------------------------------------------------------------------------------------

@@ -1295,6 +1295,12 @@ int run_backward_p1_gated(const BwdJob &j, hipStream_t s) {
     return rc;
 }
 
+// Whether p = 1 takes run_backward_p1_gated: above 64 features, but not problems of one row block each
+// way, which the narrow kernel alone ends sooner than the fill, the scan and the gated instances (both
+// directions, gated -> narrow: 64 x 64 x 101 72 -> 60 us, 600 batches of it 188 -> 112, 100 of 128 x 128 x
+// 256 131 -> 97).
+bool p1_gated(int64_t n, int64_t m, int64_t d) { return d > kBFeat && (n > kBRows || m > kBRows); }
+
 // WHOLE's conditions (lp_backward_kernel): every array's row length a multiple of 4 and the
 // staging offsets of 128 rows below 2^32 bytes.  Any alignment: the loads need a dword's.
 bool whole_loads(const BwdJob &j) {
@@ -1307,7 +1313,7 @@ template <int MODE, int PK, bool EXPG = false>
 int run_backward(const BwdJob &j, hipStream_t s) {
     const bool whole = whole_loads(j);
     if constexpr (PK == kP1 && (MODE == kRoot || MODE == kSum)) {
-        if (j.flag && j.d > kBFeat)
+        if (j.flag && p1_gated(j.n, j.m, j.d))
             return whole ? run_backward_p1_gated<MODE, EXPG, true>(j, s) : run_backward_p1_gated<MODE, EXPG, false>(j, s);
     }
     if constexpr (kWide<MODE, PK>) {
@@ -1691,16 +1697,16 @@ extern "C" int tpw_pairwise_exp_kernel_backward(const float *grad, const float *
                  nullptr, nullptr, false, out, -gamma};
         return run_backward<kSum, kP2, true>(j, s);
     }
-    // p = 1: above 64 features (run_backward_p1_gated) the gradient is formed while the kernels
+    // p = 1: where run_backward_p1_gated runs, the gradient is formed while the kernels
     // stage their pairs (the narrow fallback instance too, at two waves per SIMD: it runs
     // only for values outside the sign path's range); elsewhere a second per-pair array would
-    // take the narrow kernel from three waves per SIMD to two (156 -> 174 VGPRs), so one
+    // take the narrow kernel from three waves per SIMD to two (185 VGPRs), so one
     // elementwise pass writes the gradients into the workspace first
     {
         BwdJob j{grad, nullptr, nullptr, x1, x2, nullptr, batch, n, m, d, 1.0, grad_x1, grad_x2, nullptr, part,
                  nullptr, nullptr, false, out, -gamma};
         j.flag = lay.flag_word(ws);
-        if (d > kBFeat) return run_backward<kRoot, kP1, true>(j, s);
+        if (p1_gated(n, m, d)) return run_backward<kRoot, kP1, true>(j, s);
     }
     const int64_t len = batch * n * m;
     const bool vec = aligned16(grad) && aligned16(out) && aligned16(pair1);
