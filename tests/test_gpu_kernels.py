@@ -218,16 +218,22 @@ def test_lp_backward(p, B, n, m, d, entry):
                      what=f"lp p={p} {nm}")
 
 
-@pytest.mark.parametrize("p,d,wide", [(2.0, 70, 2), (3.0, 65, 2), (2.5, 70, 0), (4.5, 128, 0), (1.5, 128, 0),
-                                      (float("inf"), 70, 0), (3.0, 64, 0)])
-def test_lp_backward_kernel_widths(p, d, wide):
-    """Which p take the 128-feature kernel above 64 features (both directions, no other launch)."""
-    x1, x2, g = (t.to(DEV) for t in (randn(90, d, seed=1), randn(101, d, seed=2), randn(90, 101, seed=3)))
-    dist = capi.lp_distances(x1, x2, p)
+@pytest.mark.parametrize("p,m,d,wide", [(2.0, 101, 70, 2), (3.0, 101, 65, 2), (2.5, 101, 70, 0), (4.5, 100, 128, 0),
+                                        (1.5, 100, 128, 0), (float("inf"), 101, 70, 0), (3.0, 101, 64, 0),
+                                        (3.0, 100, 129, 0), (3.0, 101, 192, 0), (2.0, 100, 300, 0), (3.0, 101, 250, 2),
+                                        (3.0, 100, 388, 2), (3.0, 101, 388, 0), (3.0, 101, 450, 2)])
+def test_lp_backward_kernel_widths(p, m, d, wide):
+    """Which p and d take the 128-feature kernel above 64 features (both directions, no other launch)."""
+    n = 92
+    x1, x2, g = randn(n, d, seed=1), randn(m, d, seed=2), randn(n, m, seed=3)
+    dist = capi.lp_distances(x1.to(DEV), x2.to(DEV), p)
     for family, count in (("lp_backward_wide_kernel", wide), ("lp_backward_narrow_kernel", 2 - wide)):
         timer = capi.LaunchTimer(family, 8).arm()
-        capi.lp_distances_backward2(g, x1, x2, dist, p)
+        got = capi.lp_distances_backward2(g.to(DEV), x1.to(DEV), x2.to(DEV), dist, p)
         assert len(timer.read()[0]) == count, family
+    a, b = x1.double().requires_grad_(), x2.double().requires_grad_()
+    for t, want in zip(got, torch.autograd.grad(torch.cdist(a, b, p), (a, b), g.double())):
+        assert_close(t, want, rtol=1e-4, atol=1e-5 * float(want.abs().max()) + 1e-6, what=f"p={p} d={d}")
 
 
 def _sign_counts(a, b):
@@ -323,11 +329,11 @@ def test_lp_backward_p1_wide_gated(entry, outside):
 
 
 @pytest.mark.parametrize("B,n,m,d,launches", [(1, 64, 64, 101, 2), (1, 32, 1, 65, 2), (3, 64, 63, 128, 2),
-                                              (1, 128, 65, 101, 2), (2, 129, 64, 96, 4), (1, 5, 130, 67, 4),
-                                              (1, 200, 64, 64, 2)])
+                                              (1, 128, 200, 101, 2), (2, 129, 130, 96, 4), (1, 300, 5, 67, 2),
+                                              (1, 140, 133, 150, 2), (1, 140, 133, 193, 4), (1, 200, 164, 64, 2)])
 def test_lp_backward_p1_launches(B, n, m, d, launches):
-    """p = 1 above 64 features: problems of one row block each way take the narrow kernel's two launches
-    alone, larger ones the wide and the narrow kernel behind the range scan.  grad = 1: sign counts bit for bit."""
+    """p = 1 above 64 features: problems of one row block one way, and 129 to 192 features, take the narrow
+    kernel's two launches alone, others the wide and the narrow kernel behind the range scan.  grad = 1: sign counts bit for bit."""
     rng = np.random.default_rng(13)
     a = (rng.integers(-8, 9, size=(B, n, d)) * 0.125).astype(np.float32)
     b = (rng.integers(-8, 9, size=(B, m, d)) * 0.125).astype(np.float32)

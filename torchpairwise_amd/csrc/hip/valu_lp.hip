@@ -1295,11 +1295,24 @@ int run_backward_p1_gated(const BwdJob &j, hipStream_t s) {
     return rc;
 }
 
-// Whether p = 1 takes run_backward_p1_gated: above 64 features, but not problems of one row block each
+// Whether p = 1 takes run_backward_p1_gated: above 64 features, but not problems of one row block one
 // way, which the narrow kernel alone ends sooner than the fill, the scan and the gated instances (both
-// directions, gated -> narrow: 64 x 64 x 101 72 -> 60 us, 600 batches of it 188 -> 112, 100 of 128 x 128 x
-// 256 131 -> 97).
-bool p1_gated(int64_t n, int64_t m, int64_t d) { return d > kBFeat && (n > kBRows || m > kBRows); }
+// directions, gated -> narrow: 64 x 64 x 101 72 -> 60 us, 600 batches of it 188 -> 112, 50 of 104 x 7779 x
+// 412 3870 -> 2981), nor three 64-feature tiles, of which the wide kernel pays for four (129 to 192
+// features: 8192^2 1831 -> 1723, 3001 x 3003 341 -> 287; 288 of 4096^2 786 -> 808, so five stay).
+bool p1_gated(int64_t n, int64_t m, int64_t d) {
+    return d > kBFeat && n > kBRows && m > kBRows && cdiv(d, kBFeat) != 3;
+}
+
+// Whether the cdist backward at p = 2 and 3 takes the wide kernel above 64 features: not where an odd
+// number of 64-feature tiles leaves it a half tile to pay for, if they are three or five (p = 3, wide ->
+// narrow: 8192^2 x 160 1950 -> 1703 us, 4096^2 x 288 819 -> 745, but x 416 1000 -> 1056) or the loads are
+// not whole (104 x 7779 x 412 in 50 batches 3572 -> 2832).  The power sum, 1.3 times as fast on the
+// wide kernel, always does.
+bool wide_pays(int64_t d, bool whole) {
+    const int64_t tiles = cdiv(d, kBFeat);
+    return tiles % 2 == 0 || (whole && tiles > 5);
+}
 
 // WHOLE's conditions (lp_backward_kernel): every array's row length a multiple of 4 and the
 // staging offsets of 128 rows below 2^32 bytes.  Any alignment: the loads need a dword's.
@@ -1317,7 +1330,7 @@ int run_backward(const BwdJob &j, hipStream_t s) {
             return whole ? run_backward_p1_gated<MODE, EXPG, true>(j, s) : run_backward_p1_gated<MODE, EXPG, false>(j, s);
     }
     if constexpr (kWide<MODE, PK>) {
-        if (j.d > kBFeat)
+        if (j.d > kBFeat && (MODE == kSum || wide_pays(j.d, whole)))
             return whole ? run_backward_fw<MODE, PK, kBFeatWide, false, EXPG, true>(j, s)
                          : run_backward_fw<MODE, PK, kBFeatWide, false, EXPG, false>(j, s);
     }
