@@ -104,7 +104,7 @@ __device__ __forceinline__ void xcd_tile_of(int64_t bid, int64_t tiles_n, int64_
 }
 
 // Raw buffer resource over the `elems` floats that start at `base` (word 3 0x00020000: the
-// 32-bit data format of gfx9 raw buffers).  A dword load at a byte offset at or past the end
+// 32-bit data format of gfx9 raw buffers).  A load at byte offsets at or past the end
 // returns 0 without touching memory; elems <= 0 makes every load return 0.  The range is
 // clamped to 2^32 - 1 bytes, so lane offsets must stay below that.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_over(const float *base, int64_t elems) {
@@ -112,10 +112,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_over(const float *base,
     const uint32_t num = bytes >= (int64_t)0xffffffffLL ? 0xffffffffu : (uint32_t)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), (short)0, (int)num, 0x00020000);
 }
-__device__ __forceinline__ float buffer_load(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset) {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)byte_offset, 0, 0));
-}
-// Four floats at a dword-aligned byte offset, all of them in range.
+// Four floats at a dword-aligned byte offset, all of them in range or all past the end (zeros).
 typedef unsigned int tpw_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ floatx4 buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset) {
     return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte_offset, 0, 0));

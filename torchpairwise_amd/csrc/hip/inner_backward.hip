@@ -139,8 +139,10 @@ __device__ __forceinline__ void weight_terms(float gv, float av, float nv, float
 // The output-based cosine terms for a pair whose norms both lie in [2^-60, 2^60] (so den = n1 n2
 // is a normal nonzero float and weight_terms takes its quotient branch), from the reciprocals
 // r1 = RN(1 / n1), r2 = RN(1 / n2): gS = gq r1 r2, rt = gden n2 = -gq q r1, ct = gden n1 =
-// -gq q r2.  Within 2 ulp of weight_terms's values (which divide by the rounded n1 n2), with
-// seven VALU operations against its twenty and a reciprocal.
+// -gq q r2, with seven VALU operations against weight_terms's twenty and a reciprocal.  To first order
+// (u = 2^-24; given q) w is within 4 u of its exact value and rt, ct within 3 u, or 6 u and 4 u from reciprocals
+// within one ulp (rcp_newton's); weight_terms's, from the rounded n1 n2 and an approximate reciprocal,
+// are within 4 u and 6 u.
 template <int MODE>
 __device__ __forceinline__ void cos_terms_fast(float gv, float av, float r1, float r2, float &w, float &rt,
                                                float &ct) {
@@ -820,7 +822,8 @@ OpPlan op_plan(int64_t batch, int64_t n, int64_t m, int64_t d) {
     // Chunks of the whole launch per block slot.  Where n and m are far apart the many blocks of
     // one direction fill the chip and the few of the other would each walk the long K alone
     // (8 x 100 x 12001 x 150, euclidean forward and backward: 1268 -> 383 us), so a
-    // block takes at most one and a half shares, and eight chunks without asking.
+    // block takes at most one and a half shares, and eight chunks without asking, as far as 32
+    // splits go (100 x 250000 x 128: a share and a half is 91 chunks, a block of grad_x1 walks 245).
     const int64_t share =
         (cdiv(n, kOpRows) * cdiv(m, kOpK) + cdiv(m, kOpRows) * cdiv(n, kOpK)) * P.tiles_f * batch * 3 / (2 * fill);
     for (int t = 0; t < 2; ++t) {
