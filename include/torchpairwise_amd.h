@@ -335,9 +335,14 @@ int tpw_pairwise_inner(const void *x1, const void *x2, int dtype, int64_t batch,
 int tpw_pairwise_inner_own_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
                                  int64_t m, int64_t d, int epilogue, void *out, void *stream);
 
-/* 1 where tpw_pairwise_inner runs its small-output kernel on these operands (only the alignment
- * of x1 and x2 is looked at), which takes rows of any length and alignment at full speed; else 0.
- * Replaces no reference kernel (its norms are separate ATen calls). */
+/* 1 where tpw_pairwise_inner runs its small-output kernel on these operands at this epilogue
+ * (TPW_EPI_DOT, which sums no norms, has lines of its own; only the alignment of x1 and x2 is
+ * looked at), which takes rows of any length and alignment at full speed; else 0. */
+int tpw_pairwise_inner_is_small(const void *x1, const void *x2, int dtype, int64_t batch,
+                                int64_t n, int64_t m, int64_t d, int epilogue);
+
+/* The same at the epilogues that use norms.  Replaces no reference kernel (its norms are separate
+ * ATen calls). */
 int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch,
                                    int64_t n, int64_t m, int64_t d);
 

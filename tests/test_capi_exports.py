@@ -81,6 +81,18 @@ def test_small_output_rule():
     assert small(f32, 250, 128, 128, 1000) and small(bf16, 250, 128, 128, 3000) and small(bf16, 1, 16000, 60, 768)
     assert not small(f32, 260, 64, 64, 50) and not small(bf16, 260, 64, 64, 50)
 
+    def dot(dtype, b, n, m, d, offset=0):
+        return bool(l.tpw_pairwise_inner_is_small(4096 + offset, 8192, dtype, b, n, m, d, _capi.EPI_DOT))
+
+    # without norms (regression: the lines above, up to 1.9 times as slow here)
+    assert dot(f32, 1, 1920, 1920, 340) and dot(f32, 1, 906, 3692, 1001) and dot(f32, 14, 500, 470, 2100)
+    assert not dot(f32, 1, 1920, 1920, 1001) and not dot(f32, 1, 906, 3692, 2100) and not dot(f32, 1, 2048, 2047, 512)
+    assert dot(bf16, 1, 1024, 1024, 2048) and dot(bf16, 1, 1300, 1900, 3000) and dot(bf16, 14, 500, 470, 3000)
+    assert dot(bf16, 1, 1024, 1024, 4100) and dot(bf16, 1, 1000, 1050, 2048) and dot(bf16, 1, 1920, 1920, 2500, 2)
+    assert dot(bf16, 1, 1300, 1900, 4100) and dot(bf16, 14, 500, 470, 4001) and dot(bf16, 1, 2000, 1700, 3000)
+    assert not dot(bf16, 1, 1000, 2048, 1024) and not dot(bf16, 1, 1300, 1900, 8000) and not dot(bf16, 1, 1920, 1920, 4001)
+    assert not dot(f32, 260, 64, 64, 50) and not dot(bf16, 260, 64, 64, 50)
+
 
 def test_argument_errors_are_reported_without_gpu():
     l = _capi.lib()

@@ -50,6 +50,7 @@ _SIGNATURES = {
     "tpw_row_norms2": (_i, [_p, _i64, _p, _i64, _i, _i64, _i, _p, _p, _p]),
     "tpw_pairwise_inner": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _p, _p, _i, _p, _p]),
     "tpw_pairwise_inner_own_norms": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _i, _p, _p]),
+    "tpw_pairwise_inner_is_small": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _i]),
     "tpw_pairwise_inner_forms_norms": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64]),
     "tpw_radius_mask_euclidean": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _p, _p, C.c_float, _p, _p]),
     "tpw_pairwise_exp_kernel": (_i, [_p, _p, _i64, _i64, _i64, _i64, _i, C.c_float, _p, _p]),

@@ -1067,8 +1067,15 @@ int64_t cu_count() {
 // 56 -> 64).  Four blocks a CU pay at few features (2048^2: fp32 d = 300 45.9 -> 44.1, 500 58 -> 69;
 // bf16 500 27.6 -> 27.3, 1000 35.6 -> 39.4) or where the copies are of many rows (250 x 128 x 128
 // fp32 x 1000 248 -> 179, bf16 106 -> 50).
+// All of that is with the norms, which the small kernel sums once per block and no launch saves to
+// DOT, so that its lines lie further out.  Whole rows, bf16: one block a CU at any d (1024^2 x 2048
+// 21.6 -> 19.9), two where output rows are no whole units (1000 x 1050 x 2048 22.0 -> 21.4, but
+// 1000 x 2048 21.7 -> 22.1).  Copied rows: fp32 1920^2 x 340 46 -> 35, 700 65.0 -> 62.6, but 1001 86.9 ->
+// 89.8; 906 x 3692 x 1001 92.9 -> 90.5, but 2100 168 -> 176; 14 x 500 x 470 x 2100 201 -> 174.  bf16 1300 x
+// 1900 x 2100 44.5 -> 33, 4100 70 -> 60, odd 4001 70 -> 74; 2048^2 x 1500 41 -> 32, 2000 x 1700 x 3000
+// 59.5 -> 51.7, 4001 72 -> 84; 14 x 500 x 470 x 4001 107 -> 84.
 template <typename T>
-bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d) {
+bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, int64_t d, bool norms) {
     const int64_t cus = cu_count(), blocks = cdiv(n, kST) * cdiv(m, kST) * batch, rows = batch * (n + m);
     if (cdiv(n, kTile) * cdiv(m, kTile) * batch > cus) return false;
     constexpr bool f32 = sizeof(T) == 4;
@@ -1076,11 +1083,14 @@ bool small_fits(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, i
     const bool two = blocks <= 2 * cus, three = blocks <= 3 * cus;
     if (row16 && d % Elem<T>::kChunk == 0) {
         if (f32) return two || (three && d <= 384);
+        if (!norms && (blocks <= cus || (two && m % 8 != 0))) return true;
         const int64_t most = rows >= 8192 ? 896 : blocks <= cus && m % 8 != 0 ? 1024 : 512;
         return (three && d <= 256) || (two && d <= most);
     }
     if (!row16 && batch * n * m < ((int64_t)1 << 20)) return true;
-    if (f32) return three || d <= 320 || rows >= 16384 + 8 * d;
+    if (!norms && rows >= (f32 ? 4 : 3) * d) return true;
+    if (f32) return three || d <= (norms ? 320 : 896) || rows >= 16384 + 8 * d;
+    if (!norms) return two || d <= (three ? 4352 : 3072);
     return three ? d <= 2048 || rows >= 8192 : d <= 704 || rows >= 16384;
 }
 
@@ -1104,7 +1114,8 @@ int launch_inner(const T *x1, const T *x2, int64_t batch, int64_t n, int64_t m, 
                  const float *aux1, const float *aux2, OutT *out, hipStream_t s,
                  const OutT *X = nullptr, float sign = 1.0f, KerParams kp = {}) {
     if constexpr (EPI <= TPW_EPI_CORRELATION && std::is_same<T, OutT>::value) {
-        if (small_fits(x1, x2, batch, n, m, d)) return launch_small<T, EPI>(x1, x2, batch, n, m, d, aux1, aux2, out, s);
+        if (small_fits(x1, x2, batch, n, m, d, kAux1<EPI>))
+            return launch_small<T, EPI>(x1, x2, batch, n, m, d, aux1, aux2, out, s);
     }
     const int64_t tiles_n = cdiv(n, kTile), tiles_m = cdiv(m, kTile);
     const int64_t total = tiles_n * tiles_m * batch;
@@ -1514,14 +1525,20 @@ extern "C" int tpw_row_norms2(const void *x1, int64_t rows1, const void *x2, int
     return dtype == TPW_F32 ? run(static_cast<float *>(nullptr)) : run(static_cast<uint16_t *>(nullptr));
 }
 
-extern "C" int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
-                                              int64_t m, int64_t d) {
+extern "C" int tpw_pairwise_inner_is_small(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
+                                           int64_t m, int64_t d, int epilogue) {
     if (batch < 0 || n < 0 || m < 0 || d < 0 || (dtype != TPW_F32 && dtype != TPW_BF16)) return 0;
+    const bool norms = epilogue != TPW_EPI_DOT;
     return (dtype == TPW_F32
-                ? small_fits(static_cast<const float *>(x1), static_cast<const float *>(x2), batch, n, m, d)
-                : small_fits(static_cast<const uint16_t *>(x1), static_cast<const uint16_t *>(x2), batch, n, m, d))
+                ? small_fits(static_cast<const float *>(x1), static_cast<const float *>(x2), batch, n, m, d, norms)
+                : small_fits(static_cast<const uint16_t *>(x1), static_cast<const uint16_t *>(x2), batch, n, m, d, norms))
                ? 1
                : 0;
+}
+
+extern "C" int tpw_pairwise_inner_forms_norms(const void *x1, const void *x2, int dtype, int64_t batch, int64_t n,
+                                              int64_t m, int64_t d) {
+    return tpw_pairwise_inner_is_small(x1, x2, dtype, batch, n, m, d, TPW_EPI_EUCLIDEAN);
 }
 
 namespace {

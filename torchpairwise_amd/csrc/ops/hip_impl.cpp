@@ -94,7 +94,8 @@ at::Tensor pw_inner_cuda(const at::Tensor &x1, const at::Tensor &x2, int64_t epi
     at::Tensor n1, n2;
     void *s = current_stream();
     // small outputs: one launch, norms inside
-    const bool small = tpw_pairwise_inner_forms_norms(a.data_ptr(), b.data_ptr(), dt, B, n, m, d) != 0;
+    const bool small =
+        tpw_pairwise_inner_is_small(a.data_ptr(), b.data_ptr(), dt, B, n, m, d, static_cast<int>(epilogue)) != 0;
     if (epilogue != TPW_EPI_DOT && !small) {
         const int squared = (epilogue == TPW_EPI_EUCLIDEAN || epilogue == TPW_EPI_SQEUCLIDEAN);
         n1 = at::empty({B, n}, a.options().dtype(at::kFloat));
