@@ -1973,12 +1973,15 @@ __global__ __launch_bounds__(256, 2) void op_backward_kernel(
     int64_t tiles_f, KerParams kp, float sign, T *__restrict__ gx1, T *__restrict__ gx2, float *part1, float *coef1,
     float *part2, float *coef2) {
     __shared__ OpShared<T, FT> sh;
-    const int64_t bid = blockIdx.x;
-    if (bid < d1.blocks)
-        op_body<T, MODE, FT, false>(sh, bid, d1, tiles_f, g, res, x1, x2, n1, n2, n, m, d, kp, sign, gx1, part1, coef1);
+    // the direction of longer blocks first: behind the short ones they would end alone
+    const bool x1_first = d1.kps >= d2.kps;
+    const int64_t lead = x1_first ? d1.blocks : d2.blocks;
+    const bool leads = blockIdx.x < lead;
+    const int64_t unit = leads ? blockIdx.x : blockIdx.x - lead;
+    if (leads == x1_first)
+        op_body<T, MODE, FT, false>(sh, unit, d1, tiles_f, g, res, x1, x2, n1, n2, n, m, d, kp, sign, gx1, part1, coef1);
     else
-        op_body<T, MODE, FT, true>(sh, bid - d1.blocks, d2, tiles_f, g, res, x2, x1, n1, n2, n, m, d, kp, sign, gx2,
-                                   part2, coef2);
+        op_body<T, MODE, FT, true>(sh, unit, d2, tiles_f, g, res, x2, x1, n1, n2, n, m, d, kp, sign, gx2, part2, coef2);
 }
 
 // Both gradients from the splits' partials [batch, splits, R, d] and row terms [batch, splits, R].
