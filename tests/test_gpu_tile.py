@@ -426,6 +426,34 @@ def test_backward_paths_of_large_problems(name, kw, path, dtype):
                          what=f"{name} {path} offset={offset} grad_x{k + 1}")
 
 
+# Batches whose weight pass and products end sooner than the one-launch kernel (regression: cosine up to 1.7
+# times and bf16 of aligned sizes 1.6 times as slow on it), and their neighbours that stay; long blocks of
+# either direction first.  Bar as above.
+@pytest.mark.parametrize("name,dtype,B,n,m,d,one", [
+    ("cosine_distances", torch.float32, 50, 128, 1664, 200, 0), ("cosine_distances", torch.float32, 50, 64, 300, 200, 1),
+    ("cosine_distances", torch.bfloat16, 200, 128, 128, 427, 0), ("cosine_distances", torch.bfloat16, 50, 66, 3468, 200, 1),
+    ("linear_kernel", torch.bfloat16, 200, 128, 128, 640, 0), ("linear_kernel", torch.bfloat16, 200, 128, 127, 640, 1),
+    ("euclidean_distances", torch.bfloat16, 200, 192, 128, 384, 0), ("euclidean_distances", torch.float32, 16, 2880, 93, 427, 1),
+])
+def test_backward_batches_one_launch_or_passes(name, dtype, B, n, m, d, one):
+    import torchpairwise_amd as tp
+    from tests._util import assert_close
+
+    print(f"{name} {dtype} B={B} n={n} m={m} d={d}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(6)
+    x1, x2, g = (torch.randn(B, r, c, generator=gen, device=DEV).to(dtype) for r, c in ((n, d), (m, d), (n, m)))
+    a, b = x1.clone().requires_grad_(), x2.clone().requires_grad_()
+    out = getattr(tp, name)(a, b)
+    with Launches("op_backward_kernel") as launches:
+        got = torch.autograd.grad(out, (a, b), g)
+    assert launches.count == one
+    tol = 1e-4 if dtype == torch.float32 else 1e-2
+    for i in (0, B - 1):
+        ra, rb = x1[i].double().requires_grad_(), x2[i].double().requires_grad_()
+        for t, w in zip(got, torch.autograd.grad(_op64(name, {}, ra, rb), (ra, rb), g[i].double())):
+            assert_close(t[i].float(), w, rtol=tol, atol=tol * float(w.abs().max()), what=f"{name} batch {i}")
+
+
 # bf16 backward of small problems with aligned inputs and with inputs offset by one element
 # (polynomial: the weight pass and the products; the others: op_backward_kernel with whole and element
 # loads): bar: the bf16 tolerance against float64 autograd, 1e-2 (+ 1e-2 * max), and the two calls

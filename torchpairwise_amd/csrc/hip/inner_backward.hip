@@ -1598,8 +1598,31 @@ int products_f32(const float *W, const float *x1, const float *x2, int64_t batch
 // 8000 x 4000 x 400 946 against 1730, 16383 x 8191 x 60 1480 against 1990.  bf16 700 x 900 x 100
 // 283 -> 67, 2118 x 6656 x 128 483 -> 150, 2900 x 2901 x 200 725 -> 268, 2048^2 x 512 129 -> 95;
 // 4096^2 x 512 204 against 290, 8 x 1048 x 11312 x 191 880 against 1910.
-bool op_fits(const OpPlan &P, int64_t batch, int64_t n, int64_t m) {
-    return (double)batch * (double)n * (double)m * (double)P.tiles_f <= 3.0 * 0x1p23;
+// Cosine's weights are the dearest, and a block costs about four chunks beside its own.  With more chunks
+// so counted per block slot (load) than below the passes are ahead where they have the blocks to fill the
+// GPU (t1, t2: 128 x 128 tiles of the products).  One launch -> passes, forward and backward:
+//   fp32: 50 x 128 x 1664 x 200 292 -> 233 us, 50 x 320 x 512 x 384 268 -> 238, but 50 x 169 x 1343 x 256 309 -> 345;
+//   bf16, W and W^T in whole 16-byte rows: 200 x 128 x 128 x 512 179 -> 84, 50 x 64 x 640 x 512 120 -> 99, 1600 x
+//   2496 x 768 160 -> 115 (but 1920 x 1408 x 768 117 -> 133); fewer feature tiles or ragged d: 16 x 2432 x 192
+//   x 256 151 -> 118, 16 x 704 x 832 x 250 187 -> 132, but 16 x 320 x 3008 x 100 113 -> 168, 4 x 128 x 5312 x 700
+//   228 -> 291;
+//   bf16, others: 50 x 41 x 1016 x 427 264 -> 208, 50 x 343 x 352 x 427 374 -> 321, but 200 x 309 x 298 x 100
+//   251 -> 390, 202 x 3530 x 700 in 4 batches 189 -> 545.
+bool op_fits(const OpPlan &P, int64_t batch, int64_t n, int64_t m, int64_t d, bool cosine, bool bf16) {
+    if ((double)batch * (double)n * (double)m * (double)P.tiles_f > 3.0 * 0x1p23) return false;
+    if (!cosine) return true;
+    const int64_t cus = device_cus();
+    int64_t chunks = 0;
+    for (const OpDir &D : P.dir) chunks += D.blocks * (D.kps / kOpK + 4);
+    const double load = (double)chunks / (double)(2 * cus);
+    const int64_t per_row = batch * cdiv(d, tile::kT), t1 = cdiv(n, tile::kT) * per_row, t2 = cdiv(m, tile::kT) * per_row;
+    const int64_t most = t1 > t2 ? t1 : t2, least = t1 > t2 ? t2 : t1;
+    if (!bf16) return load <= 44 || 4 * most < 7 * cus;
+    if (n % 8 == 0 && m % 8 == 0) {
+        if (d % 8 == 0 && P.tiles_f >= 3) return load <= 32;
+        return load <= 38 || 2 * most < cus || 8 * least <= cus;
+    }
+    return load <= 50 || P.tiles_f < 3 || 4 * least <= 3 * cus;
 }
 
 // 1 / v within an ulp, for normal v in cos_norm_fast's range: the hardware reciprocal and a Newton step.
@@ -2075,7 +2098,7 @@ int run_backward(const T *g, const T *x1, const T *x2, const T *res, const float
     }
     if constexpr (MODE == kDot && !kBf16) {
         const OpPlan P = op_plan(batch, n, m, d);
-        if (op_fits(P, batch, n, m) && !tile_grid_fills(batch, n, d))
+        if (op_fits(P, batch, n, m, d, false, false) && !tile_grid_fills(batch, n, d))
             return run_op_backward<T, MODE>(P, g, x1, x2, res, n1, n2, batch, n, m, d, gx1, gx2,
                                             static_cast<float *>(ws), s, kp);
         // fp32: grad is the weight matrix as stored; no weight pass, zero coefficients
@@ -2206,9 +2229,11 @@ int run_backward(const T *g, const T *x1, const T *x2, const T *res, const float
             return check_launch("cos_proj_finish_kernel");
         }
     }
+    // (bf16 products on the tile kernel, their grids full both ways, end sooner: linear 200 x 128 x 128 x 640
+    // 104 -> 63 us, euclidean 200 x 192 x 128 x 384 91 -> 76, sigmoid 200 x 192 x 64 x 384 64 -> 61)
     if constexpr (!kCosMode && MODE != kPoly) {
         const OpPlan P = op_plan(batch, n, m, d);
-        if (op_fits(P, batch, n, m))
+        if (!bf16_kmajor && op_fits(P, batch, n, m, d, kCosO<MODE>, kBf16))
             return run_op_backward<T, MODE>(P, g, x1, x2, res, n1, n2, batch, n, m, d, gx1, gx2,
                                             static_cast<float *>(ws), s, kp);
     }
